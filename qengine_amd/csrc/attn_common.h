@@ -360,6 +360,8 @@ hipError_t launch_q8_attn_split(const AttnArgs& a, hipStream_t stream);
 hipError_t launch_q8_attn_fast(const AttnArgs& a, uint16_t* out, hipStream_t stream);
 hipError_t launch_q8k_tq3v_attn_fast(const AttnArgs& a, uint16_t* out, hipStream_t stream);
 hipError_t launch_q8_attn_fast_append(const AttnArgs& a, uint16_t* out, hipStream_t stream);
+// multi-query decode over Q8_0 keys (attn_mq.hip), values Q8_0 or TQ3
+hipError_t launch_mq_attn(const AttnArgs& a, bool v_tq3, uint16_t* out, hipStream_t stream);
 hipError_t launch_split_merge(const float* m, const float* l, const float* o, uint16_t* out,
                               int num_q, int sub_n, int sub_n_max, int k_splits,
                               hipStream_t stream);

@@ -704,6 +704,60 @@ size_t qkv_decode_attn_q8_workspace_bytes(int num_q, int num_kv, int sub_n, int 
   return fast_ws_upto(num_q, num_kv, sub_n, n_keys, kChunkKeysQ8, 0, 0);
 }
 
+// Multi-query calls over Q8_0 keys take the kernel that reads every tile once
+// for up to 64 (query, head) columns (mq_attn_kernel), unless one workgroup
+// per (kv head, query, chunk) fits the GPU in one round: then q8_attn_kernel's
+// shorter chain wins (1,000 keys, 2 to 8 queries: 9.6-9.8 us against
+// 11.6-11.8; 12 queries, 384 workgroups: 12.4 against 12.1; 4,096 keys, 2
+// queries, 272 workgroups: 13.4 against 12.6).  Two of its workgroups share a
+// CU, and with more than 4 heads per column block of the other kernel that
+// second round still wins while the chunks are few (GQA 6 over 1,000 keys, 16
+// queries: 14.2 against 15.3; over 4,096, 2 queries: 13.7 against 12.7).
+bool q8_takes_mq(const FastGeom& g, int num_q, int num_kv, int sub_n) {
+  const long round = num_q / num_kv > 4 && g.n_chunks <= 16 ? 2 * kMaxFastWgs : kMaxFastWgs;
+  return sub_n > 1 && (long)sub_n * g.n_chunks * num_kv > round;
+}
+
+// Queries per workgroup and chunks of that kernel.  Chunks are whole 64-key
+// tiles, at least two (a chunk pays for its records), and never more than in
+// `g`, the geometry that the workspace queries describe (128 keys and up per
+// chunk); the launch is one round of the GPU.  A call that leaves CUs idle is
+// split over query groups: fewer columns make a tile cheaper and leave each
+// workgroup fewer record rows to write.
+// Costs as measured: 1.8 us per tile up to 32 columns, 2.36 with 64 (16 tiles
+// per workgroup against 5), 64 KB of records per workgroup ~3.2 us.
+int mq_geom(FastGeom& g, int num_q, int num_kv, int sub_n, int n_keys) {
+  const int gqa = num_q / num_kv;
+  const int tiles = (n_keys + 63) / 64;
+  int best_qpw = 0, best_tpc = 0;
+  float best = 0.0f;
+  for (int groups = 1; groups <= sub_n; groups *= 2) {
+    const int qpw = (sub_n + groups - 1) / groups;
+    if (qpw * gqa > 64) continue;
+    const int used = (sub_n + qpw - 1) / qpw, cols = qpw * gqa;
+    const long limit = std::max<long>(1, std::min<long>(g.n_chunks, kMaxFastWgs / ((long)used * num_kv)));
+    const int tpc = (int)std::max<long>(2, (tiles + limit - 1) / limit);
+    const long wgs = (long)used * num_kv * ((tiles + tpc - 1) / tpc);
+    const float rounds = (float)((wgs + kMaxFastWgs - 1) / kMaxFastWgs);
+    const float cost = rounds * (tpc * (cols > 32 ? 2.36f : 1.8f) + 0.05f * cols);
+    if (best_qpw == 0 || cost < best) {
+      best = cost;
+      best_qpw = qpw;
+      best_tpc = tpc;
+    }
+  }
+  if (best_qpw == 0) {   // (more queries than 2^k groups of 64 columns hold)
+    best_qpw = 64 / gqa;
+    const long used = (sub_n + best_qpw - 1) / best_qpw;
+    const long limit = std::max<long>(1, std::min<long>(g.n_chunks, kMaxFastWgs / (used * num_kv)));
+    best_tpc = (int)std::max<long>(2, (tiles + limit - 1) / limit);
+  }
+  g.chunk_keys = 64 * best_tpc;
+  g.n_chunks = (tiles + best_tpc - 1) / best_tpc;
+  g.n_slots = g.n_chunks;
+  return best_qpw;
+}
+
 // Fast path over Q8_0 keys; values Q8_0 (v_tq3 false) or TQ3 (v_tq3 true).
 static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint16_t* out,
                           int num_q, int num_kv, int head_dim, int start_pos, int sub_n,
@@ -716,8 +770,10 @@ static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint1
   if (!aligned(q, 16) || !aligned(k, 4) || !aligned(v, 4) || !aligned(out, 16))
     return QKV_ERR_ALIGN;
   const int n_keys = start_pos + sub_n;
-  const FastGeom g = fast_geom(num_q, num_kv, sub_n, n_keys, kChunkKeysQ8);
+  FastGeom g = fast_geom(num_q, num_kv, sub_n, n_keys, kChunkKeysQ8);
   if (!workspace || workspace_bytes < g.total) return QKV_ERR_WORKSPACE;
+  const bool mq = q8_takes_mq(g, num_q, num_kv, sub_n);
+  const int qpw = mq ? mq_geom(g, num_q, num_kv, sub_n, n_keys) : 1;
   if (!aligned(workspace, 256)) return QKV_ERR_ALIGN;
   char* ws = static_cast<char*>(workspace);
   qkv::AttnArgs a{};
@@ -729,7 +785,7 @@ static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint1
   a.start_pos = start_pos;
   a.sub_n = sub_n;
   a.sub_n_max = sub_n;
-  a.qpw = 1;
+  a.qpw = qpw;
   {
     const uint64_t extent = (uint64_t)n_keys * num_kv * 8 * sizeof(qkv_block_q8);
     a.kv_bytes = extent;
@@ -755,6 +811,7 @@ static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint1
     a.v_w = static_cast<uint8_t*>(const_cast<void*>(v));
     return launch_status(qkv::launch_q8_attn_fast_append(a, out, stream));
   }
+  if (mq) return launch_status(qkv::launch_mq_attn(a, v_tq3, out, stream));
   return launch_status(v_tq3 ? qkv::launch_q8k_tq3v_attn_fast(a, out, stream)
                              : qkv::launch_q8_attn_fast(a, out, stream));
 }

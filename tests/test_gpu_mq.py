@@ -1,0 +1,93 @@
+"""GPU parity of the multi-query Q8_0-key decode that reads every tile once for
+up to 64 (query, head) columns: against the single-query launches of the same
+rows (query t of a call over n keys is a one-query call over its own key
+count), at the edges of tiles, chunks, column groups and query groups."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from tests._data import kv_f16, q_f16, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a, dev):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+
+
+def _both(dev, fmt, q, kb, vb, n, num_q, num_kv):
+    """(one call with every query, one call per query) as float arrays."""
+    import torch
+    from qengine_amd import kvcache
+    sub_n = q.shape[0]
+    make, call = ((kvcache.decode_attn_q8_workspace, kvcache.decode_attn_q8) if fmt == "q8" else
+                  (kvcache.decode_attn_q8k_tq3v_workspace, kvcache.decode_attn_q8k_tq3v))
+    qd = _dev(q.view(np.uint16), dev).view(torch.float16)
+    ws = make(num_q, num_kv, sub_n, n, dev)
+    one = torch.zeros((sub_n, num_q, 256), dtype=torch.float16, device=dev)
+    many = torch.zeros_like(one)
+    kw = dict(num_q=num_q, num_kv=num_kv, scale=1 / 16)
+    for _ in range(2):   # the second call finds the workspace as the first left it
+        call(qd, kb, vb, one, ws, start_pos=n - sub_n, sub_n=sub_n, **kw)
+    for t in range(sub_n):
+        call(qd[t:t + 1].contiguous(), kb, vb, many[t:t + 1], ws, start_pos=n - sub_n + t, sub_n=1, **kw)
+    torch.cuda.synchronize()
+    return one.float().cpu().numpy(), many.float().cpu().numpy()
+
+
+# Two fp16 roundings separate the paths: the probabilities (2^-11 relative, taken
+# against different reference maxima; they average out over the keys) and the
+# output (2^-11 of an element).  Per row, relative to the row's largest element:
+# 2^-11 x 2 for the outputs plus as much for the sums.
+TOL = 4 * 2.0 ** -11
+
+
+@pytest.mark.parametrize("fmt", ["q8", "mixed"])
+@pytest.mark.parametrize("n,num_q,num_kv,sub_n", [
+    (8256, 16, 4, 2),       # whole tiles
+    (8257, 16, 4, 3),       # one key past a tile
+    (8319, 24, 4, 5),       # one key short of a tile, 30 columns
+    (5000, 24, 4, 10),      # 60 columns: 4 dead ones in the last group
+    (5000, 16, 4, 16),      # 64 columns
+    (5000, 16, 4, 17),      # query groups
+    (3000, 4, 4, 64),       # GQA 1: 64 queries
+    (3000, 16, 2, 9),       # GQA 8, two kv heads
+    (33000, 8, 1, 7),       # one kv head, many chunks
+    (70, 16, 4, 70),        # no history: chunks with causal keys only, some queries see none of theirs
+    (2100, 40, 8, 40),      # GQA 5, queries past one 64-column group
+])
+def test_multi_query_matches_single_queries(dev, fmt, n, num_q, num_kv, sub_n):
+    print(f"mq {fmt} n={n} num_q={num_q} num_kv={num_kv} sub_n={sub_n}", flush=True)
+    rng = np.random.default_rng(n + num_q + sub_n)
+    kb = _dev(O.q8_encode(kv_f16(rng, n, num_kv, 256)).view(np.uint8), dev)
+    v16 = kv_f16(rng, n, num_kv, 256)
+    vb = _dev((O.q8_encode(v16) if fmt == "q8" else O.tq3_encode(v16)).view(np.uint8), dev)
+    # queries of growing magnitude: sharp rows raise their reference maximum late
+    q = (q_f16(rng, sub_n, num_q, 256).astype(np.float32) * np.linspace(0.5, 4, sub_n)[:, None, None]).astype(np.float16)
+    one, many = _both(dev, fmt, q, kb, vb, n, num_q, num_kv)
+    assert np.isfinite(many).all()
+    assert rel_err(one, many) < TOL
+
+
+@pytest.mark.parametrize("fmt,plane", [("q8", "k"), ("q8", "v"), ("mixed", "k"), ("mixed", "v")])
+def test_non_finite_rows_stay_with_the_queries_that_see_them(dev, fmt, plane):
+    """An inf in the row of key n - 6 (a row of the block itself) reaches no
+    query before it.  Later ones: an inf value row makes the same elements
+    non-finite as in single-query calls; an inf key row makes the sum of its
+    chunk NaN, and the merge drops a chunk without a positive sum, so those
+    rows depend on where the chunks lie and are not compared."""
+    n, num_q, num_kv, sub_n = 4300, 16, 4, 16
+    seen = sub_n - 6
+    rng = np.random.default_rng(5)
+    k16, v16 = kv_f16(rng, n, num_kv, 256), kv_f16(rng, n, num_kv, 256)
+    (k16 if plane == "k" else v16)[n - 6, 1, 37] = np.inf
+    kb = _dev(O.q8_encode(k16).view(np.uint8), dev)
+    vb = _dev((O.q8_encode(v16) if fmt == "q8" else O.tq3_encode(v16)).view(np.uint8), dev)
+    one, many = _both(dev, fmt, q_f16(rng, sub_n, num_q, 256), kb, vb, n, num_q, num_kv)
+    assert np.isfinite(many[:seen]).all() and np.isfinite(one[:seen]).all()
+    assert rel_err(one[:seen], many[:seen]) < TOL
+    if plane == "v":
+        bad = ~np.isfinite(many)
+        assert bad[seen:].any() and np.array_equal(bad, ~np.isfinite(one))
+        assert rel_err(np.where(bad, 0.0, one), np.where(bad, 0.0, many)) < TOL

@@ -126,11 +126,13 @@ constexpr int kLeadMaxHeads = 0xffff;
 // read as zero (the buffer range check), also for a tile that starts there.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t cache_rsrc(const void* base, uint64_t off,
                                                              uint64_t extent) {
-  const bool in = off < extent;
-  const uint64_t rem = in ? extent - off : 0;
-  char* b = const_cast<char*>(static_cast<const char*>(base)) + (in ? off : 0);
-  return __builtin_amdgcn_make_buffer_rsrc(b, 0, (uint32_t)(rem < 0xffffffffull ? rem : 0xffffffffull),
-                                           0x00020000);
+  // (64-bit distance tested by its halves: scalar compares only, where a 64-bit
+  // compare would go through the vector unit at every tile)
+  const uint64_t rem = extent - off;   // wraps where off is past the extent
+  const uint32_t hi = (uint32_t)(rem >> 32), lo = (uint32_t)rem;
+  const bool past = (int32_t)hi < 0;
+  char* b = const_cast<char*>(static_cast<const char*>(base)) + off;
+  return __builtin_amdgcn_make_buffer_rsrc(b, 0, past ? 0u : hi != 0u ? 0xffffffffu : lo, 0x00020000);
 }
 
 // ---- DPP wave reductions (result broadcast through lane 63) -------------
@@ -360,8 +362,8 @@ hipError_t launch_q8_attn_split(const AttnArgs& a, hipStream_t stream);
 hipError_t launch_q8_attn_fast(const AttnArgs& a, uint16_t* out, hipStream_t stream);
 hipError_t launch_q8k_tq3v_attn_fast(const AttnArgs& a, uint16_t* out, hipStream_t stream);
 hipError_t launch_q8_attn_fast_append(const AttnArgs& a, uint16_t* out, hipStream_t stream);
-// multi-query decode over Q8_0 keys (attn_mq.hip), values Q8_0 or TQ3
-hipError_t launch_mq_attn(const AttnArgs& a, bool v_tq3, uint16_t* out, hipStream_t stream);
+// multi-query decode (attn_mq.hip): TQ3 or Q8_0 keys, TQ3 or Q8_0 values (TQ3 with TQ3 keys)
+hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* out, hipStream_t stream);
 hipError_t launch_split_merge(const float* m, const float* l, const float* o, uint16_t* out,
                               int num_q, int sub_n, int sub_n_max, int k_splits,
                               hipStream_t stream);

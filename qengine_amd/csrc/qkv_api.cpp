@@ -491,6 +491,16 @@ struct FastGeom {
   int chunk_keys, n_chunks, n_slots;
   size_t header_off, ml_off, o_off, total;
 };
+// Workspace layout of a launch with g.n_chunks chunks: one record per q head,
+// query and chunk.
+void set_layout(FastGeom& g, int num_q, int sub_n) {
+  g.n_slots = g.n_chunks;
+  const size_t rows = (size_t)num_q * sub_n * g.n_slots;
+  g.header_off = 0;
+  g.ml_off = qkv::kWsHeaderBytes;
+  g.o_off = (g.ml_off + rows * qkv::kRecMlBytes + 255) & ~(size_t)255;
+  g.total = g.o_off + rows * 256 * sizeof(float);
+}
 // Chunks of base*tpw keys, at most 128 per (kv head, query): one record per
 // chunk and q head, merged by the designated merger workgroups.
 // Query groups of a contiguous TQ3 fast-path launch (16 / GQA queries share a
@@ -498,7 +508,7 @@ struct FastGeom {
 int tq3_fast_qpw(int num_q, int num_kv, int sub_n) {
   const int gqa = num_q / num_kv;
   // more than 16 (query, head) columns: up to 64 columns per workgroup, every
-  // tile decoded once for all of them (tq3_mq_kernel)
+  // tile read once for all of them (mq_attn_kernel)
   if (sub_n * gqa > 16) return std::min(sub_n, 64 / gqa);
   // one query group of rounded queries + remainders in the 16 MFMA columns, or,
   // when the call has more queries than that, 16 / GQA queries per group with
@@ -515,7 +525,7 @@ int tq3_groups(int num_q, int num_kv, int sub_n) {
 // over its 8 waves, so the join pays from 4 tiles per wave on (one wave takes
 // one more tile instead of every wave one more round: a 16-token verify over
 // 131,072 + 16 keys, 16 chunks of 16 tiles per wave and a 16-key tile, not 16
-// chunks of 17); tq3_mq_kernel runs a chunk's tiles one after another with all
+// chunks of 17); mq_attn_kernel runs a chunk's tiles one after another with all
 // of its waves, so one more tile never costs a round (32,768 + 16 keys: 64
 // chunks of 8 tiles, one with a ninth, not 33 chunks on half of the GPU).
 int tq3_join_min(int num_q, int num_kv, int sub_n) {
@@ -554,13 +564,7 @@ FastGeom fast_geom(int num_q, int num_kv, int sub_n, int n_keys, int base = kChu
   tpw = fit(join_min);
   g.chunk_keys = base * tpw;
   g.n_chunks = chunks(tpw);
-  g.n_slots = g.n_chunks;
-  const size_t rows = (size_t)num_q * sub_n * g.n_slots;
-  g.header_off = 0;
-  g.ml_off = qkv::kWsHeaderBytes;
-  (void)num_kv;
-  g.o_off = (g.ml_off + rows * qkv::kRecMlBytes + 255) & ~(size_t)255;
-  g.total = g.o_off + rows * 256 * sizeof(float);
+  set_layout(g, num_q, sub_n);
   return g;
 }
 
@@ -581,12 +585,65 @@ size_t fast_ws_upto(int num_q, int num_kv, int sub_n, int n_keys, int base, int 
   }
   return best;
 }
+
+// mq_attn_kernel (attn_mq.hip): queries per workgroup (returned) and chunks.
+// Chunks are whole 64-key tiles, at least two (a chunk pays for its records),
+// at most max_chunks of them; the launch is one round of the GPU.  A call that
+// leaves CUs idle is split over query groups: fewer columns make a tile cheaper
+// and leave each workgroup fewer record rows to write.
+// Costs as measured (131,072 against 65,000 keys): 1.7 us per tile up to 32
+// columns, 2.05 with 64; 64 KB of records per workgroup ~3.2 us.
+int mq_geom(FastGeom& g, int num_q, int num_kv, int sub_n, int n_keys, int max_chunks) {
+  const int gqa = num_q / num_kv;
+  const int tiles = (n_keys + 63) / 64;
+  int best_qpw = 0, best_tpc = 0;
+  float best = 0.0f;
+  auto tiles_per_chunk = [&](long groups) {
+    const long limit = std::max<long>(1, std::min<long>(max_chunks, kMaxFastWgs / (groups * num_kv)));
+    return (int)std::max<long>(2, (tiles + limit - 1) / limit);
+  };
+  for (int groups = 1; groups <= sub_n; groups *= 2) {
+    const int qpw = (sub_n + groups - 1) / groups;
+    if (qpw * gqa > 64) continue;
+    const int used = (sub_n + qpw - 1) / qpw, cols = qpw * gqa;
+    const int tpc = tiles_per_chunk(used);
+    const long wgs = (long)used * num_kv * ((tiles + tpc - 1) / tpc);
+    const float rounds = (float)((wgs + kMaxFastWgs - 1) / kMaxFastWgs);
+    const float cost = rounds * (tpc * (cols > 32 ? 2.05f : 1.7f) + 0.05f * cols);
+    if (best_qpw == 0 || cost < best) {
+      best = cost;
+      best_qpw = qpw;
+      best_tpc = tpc;
+    }
+  }
+  if (best_qpw == 0) {   // (more queries than 2^k groups of 64 columns hold)
+    best_qpw = 64 / gqa;
+    best_tpc = tiles_per_chunk((sub_n + best_qpw - 1) / best_qpw);
+  }
+  g.chunk_keys = 64 * best_tpc;
+  g.n_chunks = (tiles + best_tpc - 1) / best_tpc;
+  return best_qpw;
+}
+
+// Most chunks of a TQ3 launch of that kernel over n_keys keys (monotone in n_keys).
+int mq_tq3_chunks(int num_kv, int n_keys) {
+  const int tiles = (n_keys + 63) / 64;
+  return std::min({128, (tiles + 1) / 2, std::max(1, (int)kMaxFastWgs / num_kv)});
+}
+bool tq3_takes_mq(int num_q, int num_kv, int sub_n) { return (long)sub_n * (num_q / num_kv) > 16; }
 }  // namespace
 
 size_t qkv_decode_attn_tq3_workspace_bytes(int num_q, int num_kv, int sub_n, int n_keys) {
   if (num_q <= 0 || num_kv <= 0 || sub_n <= 0 || n_keys <= 0) return 0;
-  return fast_ws_upto(num_q, num_kv, sub_n, n_keys, kChunkKeys, tq3_groups(num_q, num_kv, sub_n),
-                      tq3_join_min(num_q, num_kv, sub_n));
+  size_t need = fast_ws_upto(num_q, num_kv, sub_n, n_keys, kChunkKeys, tq3_groups(num_q, num_kv, sub_n),
+                             tq3_join_min(num_q, num_kv, sub_n));
+  if (tq3_takes_mq(num_q, num_kv, sub_n)) {
+    FastGeom g{};
+    g.n_chunks = mq_tq3_chunks(num_kv, n_keys);
+    set_layout(g, num_q, sub_n);
+    need = std::max(need, g.total);
+  }
+  return need;
 }
 
 // The TQ3 fast path with its workspace at `workspace` (caller-owned, or the
@@ -603,8 +660,20 @@ static int decode_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block
   if (!aligned(q, 16) || !aligned(k, 4) || !aligned(v, 4) || !aligned(out, 16))
     return QKV_ERR_ALIGN;
   const int n_keys = start_pos + sub_n;
-  const FastGeom g = fast_geom(num_q, num_kv, sub_n, n_keys, kChunkKeys, tq3_groups(num_q, num_kv, sub_n),
-                               tq3_join_min(num_q, num_kv, sub_n));
+  FastGeom g = fast_geom(num_q, num_kv, sub_n, n_keys, kChunkKeys, tq3_groups(num_q, num_kv, sub_n),
+                         tq3_join_min(num_q, num_kv, sub_n));
+  int qpw = tq3_fast_qpw(num_q, num_kv, sub_n);
+  const bool mq = tq3_takes_mq(num_q, num_kv, sub_n);
+  if (mq) {
+    FastGeom m = g;
+    const int mqpw = mq_geom(m, num_q, num_kv, sub_n, n_keys, mq_tq3_chunks(num_kv, n_keys));
+    set_layout(m, num_q, sub_n);
+    // (the fixed scratch of the allocation-free call may only hold the longer chunks)
+    if (!noalloc || m.total <= qkv::kNoAllocScratchBytes) {
+      g = m;
+      qpw = mqpw;
+    }
+  }
   if (noalloc) {
     // no allocation: this device's scratch (looked up, and zero-filled on
     // `stream`, by the device's first qkv_tq3_init or first call here)
@@ -626,7 +695,7 @@ static int decode_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block
   a.start_pos = start_pos;
   a.sub_n = sub_n;
   a.sub_n_max = sub_n;
-  a.qpw = tq3_fast_qpw(num_q, num_kv, sub_n);
+  a.qpw = qpw;
   {
     const uint64_t extent = (uint64_t)n_keys * num_kv * 104;
     a.kv_bytes = extent;
@@ -654,8 +723,7 @@ static int decode_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block
     // encode area: a workgroup encodes the new rows it reads, at most
     // min(sub_n, 64)), or when it is one query (a decode step: the wave whose
     // tile holds the new key encodes it); else appended by their own launch
-    const int cols = a.qpw * (num_q / num_kv);
-    if ((cols > 16 && sub_n <= 64) || (sub_n == 1 && cols <= 8)) {
+    if (mq ? sub_n <= 64 : sub_n == 1) {
       a.k_new = k_new;
       a.v_new = v_new;
       a.k_w = reinterpret_cast<uint8_t*>(const_cast<qkv_block_tq3*>(k));
@@ -668,6 +736,7 @@ static int decode_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block
       if (e != hipSuccess) return launch_status(e);
     }
   }
+  if (mq) return launch_status(qkv::launch_mq_attn(a, true, true, out, stream));
   return launch_status(qkv::launch_tq3_attn(a, 0, out, stream));
 }
 
@@ -718,46 +787,6 @@ bool q8_takes_mq(const FastGeom& g, int num_q, int num_kv, int sub_n) {
   return sub_n > 1 && (long)sub_n * g.n_chunks * num_kv > round;
 }
 
-// Queries per workgroup and chunks of that kernel.  Chunks are whole 64-key
-// tiles, at least two (a chunk pays for its records), and never more than in
-// `g`, the geometry that the workspace queries describe (128 keys and up per
-// chunk); the launch is one round of the GPU.  A call that leaves CUs idle is
-// split over query groups: fewer columns make a tile cheaper and leave each
-// workgroup fewer record rows to write.
-// Costs as measured: 1.8 us per tile up to 32 columns, 2.36 with 64 (16 tiles
-// per workgroup against 5), 64 KB of records per workgroup ~3.2 us.
-int mq_geom(FastGeom& g, int num_q, int num_kv, int sub_n, int n_keys) {
-  const int gqa = num_q / num_kv;
-  const int tiles = (n_keys + 63) / 64;
-  int best_qpw = 0, best_tpc = 0;
-  float best = 0.0f;
-  for (int groups = 1; groups <= sub_n; groups *= 2) {
-    const int qpw = (sub_n + groups - 1) / groups;
-    if (qpw * gqa > 64) continue;
-    const int used = (sub_n + qpw - 1) / qpw, cols = qpw * gqa;
-    const long limit = std::max<long>(1, std::min<long>(g.n_chunks, kMaxFastWgs / ((long)used * num_kv)));
-    const int tpc = (int)std::max<long>(2, (tiles + limit - 1) / limit);
-    const long wgs = (long)used * num_kv * ((tiles + tpc - 1) / tpc);
-    const float rounds = (float)((wgs + kMaxFastWgs - 1) / kMaxFastWgs);
-    const float cost = rounds * (tpc * (cols > 32 ? 2.36f : 1.8f) + 0.05f * cols);
-    if (best_qpw == 0 || cost < best) {
-      best = cost;
-      best_qpw = qpw;
-      best_tpc = tpc;
-    }
-  }
-  if (best_qpw == 0) {   // (more queries than 2^k groups of 64 columns hold)
-    best_qpw = 64 / gqa;
-    const long used = (sub_n + best_qpw - 1) / best_qpw;
-    const long limit = std::max<long>(1, std::min<long>(g.n_chunks, kMaxFastWgs / (used * num_kv)));
-    best_tpc = (int)std::max<long>(2, (tiles + limit - 1) / limit);
-  }
-  g.chunk_keys = 64 * best_tpc;
-  g.n_chunks = (tiles + best_tpc - 1) / best_tpc;
-  g.n_slots = g.n_chunks;
-  return best_qpw;
-}
-
 // Fast path over Q8_0 keys; values Q8_0 (v_tq3 false) or TQ3 (v_tq3 true).
 static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint16_t* out,
                           int num_q, int num_kv, int head_dim, int start_pos, int sub_n,
@@ -773,7 +802,8 @@ static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint1
   FastGeom g = fast_geom(num_q, num_kv, sub_n, n_keys, kChunkKeysQ8);
   if (!workspace || workspace_bytes < g.total) return QKV_ERR_WORKSPACE;
   const bool mq = q8_takes_mq(g, num_q, num_kv, sub_n);
-  const int qpw = mq ? mq_geom(g, num_q, num_kv, sub_n, n_keys) : 1;
+  const int qpw = mq ? mq_geom(g, num_q, num_kv, sub_n, n_keys, g.n_chunks) : 1;
+  g.n_slots = g.n_chunks;
   if (!aligned(workspace, 256)) return QKV_ERR_ALIGN;
   char* ws = static_cast<char*>(workspace);
   qkv::AttnArgs a{};
@@ -811,7 +841,7 @@ static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint1
     a.v_w = static_cast<uint8_t*>(const_cast<void*>(v));
     return launch_status(qkv::launch_q8_attn_fast_append(a, out, stream));
   }
-  if (mq) return launch_status(qkv::launch_mq_attn(a, v_tq3, out, stream));
+  if (mq) return launch_status(qkv::launch_mq_attn(a, false, v_tq3, out, stream));
   return launch_status(v_tq3 ? qkv::launch_q8k_tq3v_attn_fast(a, out, stream)
                              : qkv::launch_q8_attn_fast(a, out, stream));
 }

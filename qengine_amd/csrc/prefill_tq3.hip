@@ -27,21 +27,27 @@
 //                         the value MFMA consumes.  The history is padded to a
 //                         multiple of 64 rows, the chunk follows; pad rows are
 //                         zero.
-//   prefill_attn_kernel   one workgroup per (kv head, 64 query tokens, key
-//                         split) -- two per kv head for GQA 6, three heads
-//                         each -- and one wave per (query head, 32 tokens);
-//                         chunks of at most 32 tokens take 32-token
-//                         workgroups, two per CU.  Per 32-key tile (keys
+//   prefill_attn_kernel   one workgroup per (kv head, 64 or 32 query tokens, key
+//                         segment) -- two per kv head for GQA 6, three heads
+//                         each -- and one wave per (query head, 32 tokens).
+//                         Token count and segments by prefill_schedule: 64-token
+//                         workgroups move half the L2 -> LDS bytes per MFMA and
+//                         serve full chips (2,048 tokens over 131,072: 3.94
+//                         against 4.23-4.41 ms), 32-token ones have twice the
+//                         parallelism without partials (777 tokens, no history,
+//                         GQA 6: 37 against 45 us).  Per 32-key tile (keys
 //                         [key][dim], values [dim][key] in LDS, shared by the
-//                         64 x GQA query rows of the workgroup):
+//                         query rows of the workgroup):
 //                           S^T  = K Q^T       v_mfma_f32_32x32x16_f16, M = keys
 //                           O^T += V^T P^T     M = dims, N = query tokens
 //                         so every lane owns one query row (token lane % 32)
 //                         for the softmax and the accumulators.  Workgroups
 //                         that stream the same tiles run on one XCD (shared L2).
-//   prefill_merge_kernel  merges the key splits (log-sum-exp) and stores fp16
-//                         (prefill_merge_wide_kernel when there are many splits).
+//   prefill_merge_kernel  merges the key segments (log-sum-exp) and stores fp16
+//                         (prefill_merge_wide_kernel when there are many); rows
+//                         of one segment are stored by the attention.
 #include <algorithm>
+#include <cmath>
 
 #include "qkv_device.h"
 #include "attn_common.h"
@@ -56,13 +62,6 @@ constexpr int kHD = 256;
 constexpr int kKeys = 64;                 // row granule of the staged K / V (stage tiles)
 constexpr int kTK = 32;                   // keys per attention tile
 constexpr int kWaveToks = 32;             // query tokens per wave (the MFMA N dimension)
-
-// Token groups of a workgroup: two (64 tokens, 8 waves at GQA 4, one
-// workgroup per CU) when the chunk has more than 32 tokens, else one (two
-// workgroups per CU).  Every tile a workgroup loads serves all its query rows,
-// so 64-token workgroups move half the L2 -> LDS bytes per MFMA of 32-token
-// ones (config 5(i): 3.94 against 4.23-4.41 ms per chunk, bit-identical).
-__host__ __device__ inline int prefill_token_groups(int n_tok) { return n_tok > kWaveToks ? 2 : 1; }
 
 // LDS of the attention (bytes): two tile buffers, each keys [32][512 B] then
 // values [256 dims][64 B]; 64 KB per workgroup, so two one-group workgroups
@@ -89,23 +88,35 @@ __device__ __forceinline__ int value_pos(int key32) {
   return 16 * (a >> 1) + 8 * h + 4 * (a & 1) + c;
 }
 
-// Placement of the attention workgroups: the qtiles of one pair (kv head,
-// head group, key split) stream the same tiles, so they go to consecutive
-// slots of `span` XCDs (a power of two, 32 slots -- one per CU -- each);
-// workgroup L runs on XCD L % 8.
-struct Placement {
-  int span, per, pairs_per_round, subs;
+// Attention workgroups: one per (pair, query tile, key segment), a pair being a kv
+// head and head group.  Query tile qt (32 tok_groups tokens) attends total(qt)
+// 32-key tiles -- the history's, then the chunk's own up to its last token -- in
+// ns(qt) segments of at most seg_tiles each, as equal as whole tiles allow.  The
+// list runs segment by segment, pair by pair, query tile by query tile, and each
+// XCD takes a contiguous eighth of it (workgroup L runs on XCD L % 8), so that
+// workgroups that stream the same tiles share an L2.
+struct Sched {
+  int tg, T, th, ct, qtiles, pairs;   // ct: 32-key tiles of the chunk (0: all keys in the cache)
+  __host__ __device__ Sched(const PrefillArgs& p, int heads_per_wg)
+      : tg(p.tok_groups), T(p.seg_tiles), th(p.h_pad / 32), ct(p.from_cache ? 0 : (p.n_tok + 31) / 32),
+        qtiles((p.n_tok + 32 * p.tok_groups - 1) / (32 * p.tok_groups)),
+        pairs(p.num_kv * (p.num_q / p.num_kv / heads_per_wg)) {}
+  __host__ __device__ int total(int qt) const { return th + (ct < (qt + 1) * tg ? ct : (qt + 1) * tg); }
+  __host__ __device__ int segs(int qt) const { return (total(qt) + T - 1) / T; }
+  // first query tile with more than z segments (total(qt) > z T), qtiles if none
+  __host__ __device__ int first(int z) const {
+    const long need = (long)z * T + 1 - th;
+    if (need <= 0) return 0;
+    return need > ct ? qtiles : (int)((need + tg - 1) / tg) - 1;
+  }
+  __host__ __device__ long count() const {   // workgroups
+    const int full = segs(0), last = segs(qtiles - 1);
+    long n = (long)full * qtiles;
+    for (int z = full; z < last; z++) n += qtiles - first(z);
+    return n * pairs;
+  }
 };
-__host__ __device__ inline Placement placement(int qtiles, int pairs) {
-  int want = (qtiles + 31) / 32, span = 1;
-  while (span < want && span < 8) span *= 2;
-  Placement pl;
-  pl.span = span;
-  pl.per = (qtiles + span - 1) / span;
-  pl.pairs_per_round = 8 / span;
-  pl.subs = (pairs + pl.pairs_per_round - 1) / pl.pairs_per_round;
-  return pl;
-}
+__host__ __device__ inline int prefill_heads(int gqa) { return gqa == 6 ? 3 : 4; }   // per workgroup
 
 }  // namespace
 
@@ -173,13 +184,83 @@ __global__ __launch_bounds__(256) void prefill_stage_kernel(PrefillArgs p, const
   }
 }
 
+// The same for few tiles (a short prompt's chunk, a short history): one workgroup
+// per (kv head, 32-row tile, tensor), whose four rounds of loads are all issued
+// before the first is used -- with few workgroups the loop above is sixteen
+// memory round trips in a row (13 tiles x 4 heads: 10.9 us, here 4.4).
+constexpr int kStSmallPitch = 68;   // bytes per staged value dim row (32 keys fp16 + 4)
+
+__global__ __launch_bounds__(256) void prefill_stage_small_kernel(PrefillArgs p, const uint16_t* k,
+                                                                  const uint16_t* v) {
+  __shared__ __attribute__((aligned(16))) uint8_t vt_lds[kHD * kStSmallPitch];
+  __shared__ float cent[8];
+  const int tid = threadIdx.x, part = tid & 15;
+  const long rows = (long)p.h_pad + p.n_pad;
+  const int tiles = (int)(rows / kTK);
+  const int tv = blockIdx.x & 1, ht = blockIdx.x >> 1;
+  const int h = ht / tiles, tile = ht - h * tiles;
+  const bool hist = tile * kTK < p.h_pad;   // (h_pad is whole tiles)
+  // unit u = tid / 16 + 16 i: row u / 2 of the tile, block u % 2
+  const int blk = (tid >> 4) & 1, dim0 = blk * 128 + part * 8;
+  Tq3Group gr[4];
+  uint4 raw[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int row = tile * kTK + (tid >> 5) + 8 * i;
+    if (hist) {   // (a row past the history re-reads its last row and is zeroed below)
+      const int hr = min(row, p.hist - 1);
+      gr[i] = tq3_group_load(reinterpret_cast<const uint8_t*>(tv ? p.v_cache : p.k_cache) +
+                                 ((uint64_t)(uint32_t)hr * (uint32_t)p.num_kv + h) * 104u + blk * 52u, part);
+    } else {
+      const int cr = min(row - p.h_pad, p.n_tok - 1);
+      raw[i] = *reinterpret_cast<const uint4*>((tv ? v : k) + ((long)cr * p.num_kv + h) * kHD + dim0);
+    }
+  }
+  tq3_centroid_table(cent, tid);
+  const Tq3LaneConst lc = tq3_lane_const(part);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int r = (tid >> 5) + 8 * i, row = tile * kTK + r;
+    uint32_t pk[4];
+    if (hist) {
+      tq3_group_dequant(gr[i], part, cent, lc, pk);
+    } else {
+      pk[0] = raw[i].x;
+      pk[1] = raw[i].y;
+      pk[2] = raw[i].z;
+      pk[3] = raw[i].w;
+    }
+    if (hist ? row >= p.hist : row - p.h_pad >= p.n_tok) pk[0] = pk[1] = pk[2] = pk[3] = 0u;   // pad rows
+    if (!tv) {
+      *reinterpret_cast<uint4*>(p.kx + ((long)h * rows + row) * kHD + dim0) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+    } else {
+      const int pos = value_pos(r);
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        *reinterpret_cast<uint16_t*>(vt_lds + (dim0 + e) * kStSmallPitch + pos * 2) =
+            (uint16_t)((pk[e >> 1] >> (16 * (e & 1))) & 0xffffu);
+    }
+  }
+  if (!tv) return;   // (uniform)
+  __syncthreads();
+  uint4* dst = reinterpret_cast<uint4*>(p.vt + ((long)h * tiles + tile) * kHD * kTK);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {   // 256 dims x 64 bytes
+    const int piece = i * 256 + tid;
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(vt_lds + (piece >> 2) * kStSmallPitch + (piece & 3) * 16);
+    dst[piece] = make_uint4(src[0], src[1], src[2], src[3]);
+  }
+}
+constexpr long kStSmallWgs = 512;   // 64-row tiles x kv heads up to which the small form is launched
+
 // ---------------------------------------------------------------------------
 // attention: 1-D grid (placement above); WAVES query heads of one kv head and
 // TG groups of 32 query tokens per workgroup, one wave per (head, group)
 // ---------------------------------------------------------------------------
 template <int WAVES, int TG, bool FROM_CACHE>
 __global__ __launch_bounds__(64 * WAVES * TG, TG == 1 ? 2 : 1) void prefill_attn_kernel(
-    PrefillArgs p, const uint16_t* q) {
+    PrefillArgs p, const uint16_t* q, uint16_t* out) {
   constexpr int kToks = kWaveToks * TG;   // query tokens per workgroup
   __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
   const int tid = threadIdx.x;
@@ -190,35 +271,44 @@ __global__ __launch_bounds__(64 * WAVES * TG, TG == 1 ? 2 : 1) void prefill_attn
   const int tok = lane & 31;         // query token (MFMA N index) of this lane
   const int gqa = p.num_q / p.num_kv;
   const int groups = gqa / WAVES;            // workgroups per kv head
-  const int qtiles = (p.n_tok + kToks - 1) / kToks;
-  const int pairs = p.num_kv * groups * p.n_split;
+  const Sched sc(p, WAVES);
 
-  // ---- (pair, qtile) of this workgroup
-  int pair, qt;
+  // ---- (segment z, pair, query tile) of this workgroup: entry i of the list
+  int z, pair, qt;
   {
-    const Placement pl = placement(qtiles, pairs);
-    const int L = blockIdx.x, xcd = L & 7, r = L >> 3;
-    const int sub = r / pl.per, j = r - sub * pl.per;
-    pair = sub * pl.pairs_per_round + xcd / pl.span;
-    qt = (xcd % pl.span) * pl.per + j;
-    if (qt >= qtiles || pair >= pairs || xcd / pl.span >= pl.pairs_per_round) return;
+    const int per = (int)gridDim.x >> 3;
+    int i = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    const int full = sc.segs(0), n_full = full * sc.pairs * sc.qtiles;   // segments of every query tile
+    if (i < n_full) {
+      z = i / (sc.pairs * sc.qtiles);
+      i -= z * sc.pairs * sc.qtiles;
+      pair = i / sc.qtiles;
+      qt = i - pair * sc.qtiles;
+    } else {
+      i -= n_full;
+      const int last = sc.segs(sc.qtiles - 1);
+      int c = 0, q0 = 0;
+      for (z = full; z < last; z++) {
+        q0 = sc.first(z);
+        c = sc.qtiles - q0;
+        if (i < c * sc.pairs) break;
+        i -= c * sc.pairs;
+      }
+      if (z >= last) return;   // past the end of the list
+      pair = i / c;
+      qt = q0 + (i - pair * c);
+    }
   }
-  const int z = pair % p.n_split;
-  const int hg_all = pair / p.n_split;                 // kv head * groups + head group
-  const int h = hg_all / groups, hg = hg_all - h * groups;
+  const int h = pair / groups, hg = pair - h * groups;
   const int t0 = qt * kToks;
-  const int n_q = min(kToks, p.n_tok - t0);
   const int t0w = t0 + kWaveToks * tg;              // this wave's first token
   const int n_qw = min(kWaveToks, p.n_tok - t0w);   // <= 0: a group past the last token
   const int qh = h * gqa + hg * WAVES + wave;
 
   // 32-key tiles: history rows [0, h_pad) then (unless every key comes from
   // the cache) the chunk's own keys [0, t0 + n_q)
-  const int th = p.h_pad / kTK;
-  const int tc = FROM_CACHE ? 0 : (t0 + n_q + kTK - 1) / kTK;
-  const int total = th + tc;
-  const int tps = (total + p.n_split - 1) / p.n_split;
-  const int tlo = min(total, z * tps), thi = min(total, tlo + tps);
+  const int th = sc.th, total = sc.total(qt), ns = sc.segs(qt);
+  const int tlo = (int)((long)z * total / ns), thi = (int)((long)(z + 1) * total / ns);
   const long rows = (long)p.h_pad + p.n_pad;
 
   // ---- query of (token t0 + tok, head qh): B operands, slice s of block b
@@ -377,12 +467,25 @@ __global__ __launch_bounds__(64 * WAVES * TG, TG == 1 ? 2 : 1) void prefill_attn
     }
   }
 
-  // ---------------- partials of this split: m (log2 units), l, o
+  // ---------------- partials of this segment: m (log2 units), l, o
   {
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
     lsum = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
-  if (tok < n_qw) {
+  if (ns == 1) {   // the row's only segment: its output
+    if (tok < n_qw) {
+      const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+      uint16_t* o = out + ((long)(t0w + tok) * p.num_q + qh) * kHD;
+#pragma unroll
+      for (int d = 0; d < 8; d++)
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+          const f4_t x = f4_t{acc[d][4 * a], acc[d][4 * a + 1], acc[d][4 * a + 2], acc[d][4 * a + 3]} * inv;
+          *reinterpret_cast<uint2*>(o + d * 32 + 8 * a + 4 * hh) =
+              make_uint2(f2h(x[0]) | (f2h(x[1]) << 16), f2h(x[2]) | (f2h(x[3]) << 16));
+        }
+    }
+  } else if (tok < n_qw) {
     const long row = ((long)z * p.n_tok + t0w + tok) * p.num_q + qh;
     float* po = p.part_o + row * kHD;
 #pragma unroll
@@ -398,19 +501,25 @@ __global__ __launch_bounds__(64 * WAVES * TG, TG == 1 ? 2 : 1) void prefill_attn
 // ---------------------------------------------------------------------------
 // merge of the key splits and fp16 store: 32 threads per row, 8 dims each
 // ---------------------------------------------------------------------------
+// key segments of row t * num_q + qh
+__device__ __forceinline__ int row_segs(const PrefillArgs& p, long row) {
+  return Sched(p, prefill_heads(p.num_q / p.num_kv)).segs((uint32_t)row / (uint32_t)p.num_q / (uint32_t)(32 * p.tok_groups));
+}
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs p, uint16_t* out) {
   const long row = (long)blockIdx.x * 8 + (threadIdx.x >> 5);   // t * num_q + qh
   if (row >= (long)p.n_tok * p.num_q) return;
   const int d0 = (threadIdx.x & 31) * 8;
   const long nrows = (long)p.n_tok * p.num_q;
+  const int ns = row_segs(p, row);
+  if (ns == 1) return;   // stored by the attention
   float M = -INFINITY;
-  for (int z = 0; z < p.n_split; z++) {
+  for (int z = 0; z < ns; z++) {
     const f2_t ml = *reinterpret_cast<const f2_t*>(p.part_ml + 2 * (z * nrows + row));
     if (ml[1] > 0.f) M = fmaxf(M, ml[0]);
   }
   float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float L = 0.f;
-  for (int z = 0; z < p.n_split; z++) {
+  for (int z = 0; z < ns; z++) {
     const f2_t ml = *reinterpret_cast<const f2_t*>(p.part_ml + 2 * (z * nrows + row));
     if (!(ml[1] > 0.f)) continue;
     const float w = __builtin_amdgcn_exp2f(ml[0] - M);
@@ -447,8 +556,10 @@ __global__ __launch_bounds__(256) void prefill_merge_wide_kernel(PrefillArgs p, 
   const long row = blockIdx.x;   // t * num_q + qh
   const long nrows = (long)p.n_tok * p.num_q;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ns = row_segs(p, row);
+  if (ns == 1) return;   // stored by the attention
   float m = -INFINITY;
-  for (int z = tid; z < p.n_split; z += 256) {
+  for (int z = tid; z < ns; z += 256) {
     const f2_t ml = *reinterpret_cast<const f2_t*>(p.part_ml + 2 * (z * nrows + row));
     if (ml[1] > 0.f) m = fmaxf(m, ml[0]);
   }
@@ -457,7 +568,7 @@ __global__ __launch_bounds__(256) void prefill_merge_wide_kernel(PrefillArgs p, 
   __syncthreads();
   const float M = fmaxf(fmaxf(stat[0][0], stat[0][1]), fmaxf(stat[0][2], stat[0][3]));
   float l = 0.f;
-  for (int z = tid; z < p.n_split; z += 256) {
+  for (int z = tid; z < ns; z += 256) {
     const f2_t ml = *reinterpret_cast<const f2_t*>(p.part_ml + 2 * (z * nrows + row));
     const float w = ml[1] > 0.f ? __builtin_amdgcn_exp2f(ml[0] - M) : 0.f;
     w_s[z] = w;
@@ -470,7 +581,7 @@ __global__ __launch_bounds__(256) void prefill_merge_wide_kernel(PrefillArgs p, 
   const int sg = tid >> 5, d0 = (tid & 31) * 8;
   float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-  for (int z = sg; z < p.n_split; z += 8) {
+  for (int z = sg; z < ns; z += 8) {
     const float w = w_s[z];
     const float* po = p.part_o + (z * nrows + row) * kHD + d0;
     const f4_t a = *reinterpret_cast<const f4_t*>(po);
@@ -507,14 +618,14 @@ PrefillGeom prefill_geom(int num_q, int num_kv, int n_tok, int start_pos) {
   // history rows: start_pos (prefill) or start_pos + n_tok (verify), padded to
   // whole tiles; the workspace covers the larger of the two
   g.h_pad = (start_pos + n_tok + kKeys - 1) / kKeys * kKeys;
-  const int tg = prefill_token_groups(n_tok);
+  const int tg = n_tok > kWaveToks ? 2 : 1;
   const int qtiles = (n_tok + kWaveToks * tg - 1) / (kWaveToks * tg);
   const int wgs = num_kv * (num_q / num_kv == 6 ? 2 : 1) * qtiles;
   const int tiles = g.h_pad / kKeys + g.n_pad / kKeys;
   const int slots = tg == 2 ? 256 : 512;          // workgroups of one round: 256 CUs
   int ns = (slots + wgs - 1) / wgs;
   ns = std::min(ns, std::max(1, tiles / 8));      // at least ~8 tiles per split
-  g.n_split = std::max(1, ns);
+  g.max_split = std::max(1, ns);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t at = off;
@@ -524,48 +635,107 @@ PrefillGeom prefill_geom(int num_q, int num_kv, int n_tok, int start_pos) {
   const size_t rows = (size_t)g.h_pad + g.n_pad;
   g.kx_off = take((size_t)num_kv * rows * kHD * 2);
   g.vt_off = take((size_t)num_kv * rows * kHD * 2);
-  g.ml_off = take((size_t)g.n_split * n_tok * num_q * 2 * 4);
-  g.o_off = take((size_t)g.n_split * n_tok * num_q * kHD * 4);
+  g.ml_off = take((size_t)g.max_split * n_tok * num_q * 2 * 4);
+  g.o_off = take((size_t)g.max_split * n_tok * num_q * kHD * 4);
   g.total = off;
   return g;
 }
 
-hipError_t launch_prefill_tq3(const PrefillArgs& a, int gqa, const uint16_t* q, const uint16_t* k,
+// Token groups and segments.  Times as measured on the attention alone (us per
+// 32-key tile of a workgroup): one token group 0.93-1.06 with a CU of its own, 1.88
+// with two workgroups on the CU; two groups 1.21 on an idle chip, 1.47 with 200
+// workgroups, 1.79 with 256 (clock and L2).  Partials are written and read back
+// through the memory-side cache at ~8 TB/s; rows of one segment have none, and
+// without any the merge's launch goes too.  Candidates per token-group count: one
+// segment, and the most that still run in one round (of 256 workgroups, or 512 of
+// one group) -- just past a round every CU waits for a second one (10,000 + 777
+// tokens, GQA 4: 254 us with 260 workgroups, 178 with 208; 131,072 + 300: 1,214
+// and 870).
+void prefill_schedule(PrefillArgs& a, int max_split) {
+  const int heads = prefill_heads(a.num_q / a.num_kv);
+  double best = 0.0;
+  a.tok_groups = 0;
+  for (int tg = 1; tg <= (a.n_tok > kWaveToks ? 2 : 1); tg++) {
+    PrefillArgs c = a;
+    c.tok_groups = tg;
+    c.seg_tiles = 1;
+    const Sched one(c, heads);
+    const int most = one.total(one.qtiles - 1);
+    // the longest row in at most ns segments
+    auto with = [&](int ns) {
+      c.seg_tiles = (most + ns - 1) / ns;
+      return Sched(c, heads);
+    };
+    auto consider = [&](int ns) {
+      const Sched s = with(ns);
+      const double n = (double)s.count(), load = std::min(1.0, n / 256.0);
+      double t;
+      if (tg == 2)
+        t = std::ceil(n / 256.0) * (1.2 + 0.6 * load * load);
+      else
+        t = n <= 256.0 ? 0.95 + 0.1 * load * load : std::ceil(n / 512.0) * 1.88;
+      t *= s.T;
+      const int segs = s.segs(s.qtiles - 1);
+      if (segs > 1)
+        t += 4.0 + 2.0 * (n - (double)s.qtiles * s.pairs) / (double)(segs - 1) * segs * (32.0 * tg * heads * 1024.0) /
+                       8.0e6;
+      if (a.tok_groups == 0 || t < best) {
+        best = t;
+        a.tok_groups = tg;
+        a.seg_tiles = s.T;
+        a.n_split = segs;
+      }
+    };
+    consider(1);
+    for (int round = 256; round <= (tg == 1 ? 512 : 256); round += 256) {
+      int lo = 1, hi = max_split;   // most segments with at most `round` workgroups
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if (with(mid).count() <= round) lo = mid;
+        else hi = mid - 1;
+      }
+      if (lo > 1) consider(lo);
+    }
+  }
+}
+
+hipError_t launch_prefill_tq3(const PrefillArgs& a, int max_split, int gqa, const uint16_t* q, const uint16_t* k,
                               const uint16_t* v, uint16_t* out, hipStream_t stream) {
+  // (the partial area holds max_split segments per row)
+  if ((gqa != 4 && gqa != 6) || a.n_split > max_split) return hipErrorInvalidValue;
   {
     const long tiles = ((long)a.h_pad + a.n_pad) / kKeys;
-    hipLaunchKernelGGL(prefill_stage_kernel, dim3((unsigned)(a.num_kv * tiles)), dim3(256), 0,
-                       stream, a, k, v);
+    if (a.num_kv * tiles <= kStSmallWgs)
+      hipLaunchKernelGGL(prefill_stage_small_kernel, dim3((unsigned)(4 * a.num_kv * tiles)), dim3(256), 0, stream, a,
+                         k, v);
+    else
+      hipLaunchKernelGGL(prefill_stage_kernel, dim3((unsigned)(a.num_kv * tiles)), dim3(256), 0, stream, a, k, v);
   }
-  const int tg = prefill_token_groups(a.n_tok);
-  const int qtiles = (a.n_tok + kWaveToks * tg - 1) / (kWaveToks * tg);
-  const int groups = gqa == 6 ? 2 : 1;
-  const Placement pl = placement(qtiles, a.num_kv * groups * a.n_split);
-  const dim3 grid((unsigned)(8 * pl.subs * pl.per));
-  if (gqa != 4 && gqa != 6) return hipErrorInvalidValue;
   // GQA 6: two workgroups of three heads per kv head
-  const int heads = gqa == 6 ? 3 : 4;
+  const int heads = prefill_heads(gqa), tg = a.tok_groups;
+  const dim3 grid((unsigned)((Sched(a, heads).count() + 7) / 8 * 8));
   const dim3 block((unsigned)(64 * heads * tg));
   if (tg == 2) {
     if (gqa == 4 && !a.from_cache)
-      hipLaunchKernelGGL((prefill_attn_kernel<4, 2, false>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<4, 2, false>), grid, block, 0, stream, a, q, out);
     else if (gqa == 4)
-      hipLaunchKernelGGL((prefill_attn_kernel<4, 2, true>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<4, 2, true>), grid, block, 0, stream, a, q, out);
     else if (!a.from_cache)
-      hipLaunchKernelGGL((prefill_attn_kernel<3, 2, false>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<3, 2, false>), grid, block, 0, stream, a, q, out);
     else
-      hipLaunchKernelGGL((prefill_attn_kernel<3, 2, true>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<3, 2, true>), grid, block, 0, stream, a, q, out);
   } else {
     if (gqa == 4 && !a.from_cache)
-      hipLaunchKernelGGL((prefill_attn_kernel<4, 1, false>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<4, 1, false>), grid, block, 0, stream, a, q, out);
     else if (gqa == 4)
-      hipLaunchKernelGGL((prefill_attn_kernel<4, 1, true>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<4, 1, true>), grid, block, 0, stream, a, q, out);
     else if (!a.from_cache)
-      hipLaunchKernelGGL((prefill_attn_kernel<3, 1, false>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<3, 1, false>), grid, block, 0, stream, a, q, out);
     else
-      hipLaunchKernelGGL((prefill_attn_kernel<3, 1, true>), grid, block, 0, stream, a, q);
+      hipLaunchKernelGGL((prefill_attn_kernel<3, 1, true>), grid, block, 0, stream, a, q, out);
   }
   const long rows = (long)a.n_tok * a.num_q;
+  if (a.n_split == 1) return hipGetLastError();   // (every row stored by the attention)
   if (a.n_split > kMergeMaxSplits) return hipErrorInvalidValue;
   if (a.n_split >= 16)   // one workgroup per row, the splits spread over its threads
     hipLaunchKernelGGL(prefill_merge_wide_kernel, dim3((unsigned)rows), dim3(256), 0, stream, a, out);

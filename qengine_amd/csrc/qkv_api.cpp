@@ -1048,10 +1048,10 @@ int qkv_prefill_attn_tq3(const uint16_t* q, const qkv_block_tq3* k_cache,
   a.hist = from_cache ? start_pos + n_tok : start_pos;
   a.h_pad = (a.hist + 63) / 64 * 64;
   a.n_pad = from_cache ? 0 : g.n_pad;   // no chunk rows to stage
-  a.n_split = g.n_split;
   a.from_cache = from_cache ? 1 : 0;
+  qkv::prefill_schedule(a, g.max_split);
   a.scale_log2 = scale * qkv::kLog2e;
-  return launch_status(qkv::launch_prefill_tq3(a, gqa, q, k_chunk, v_chunk, out, stream));
+  return launch_status(qkv::launch_prefill_tq3(a, g.max_split, gqa, q, k_chunk, v_chunk, out, stream));
 }
 
 }  // extern "C"

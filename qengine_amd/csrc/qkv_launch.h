@@ -101,16 +101,22 @@ struct PrefillArgs {
   int hist;                  // cache rows attended: start_pos, or start_pos + n_tok (verify)
   int h_pad;                 // hist rounded up to 64
   int n_pad;                 // chunk rows staged: n_tok rounded up to 64, 0 in verify mode
-  int n_split;
+  int tok_groups;            // 32-token groups of an attention workgroup: 1 or 2
+  int seg_tiles;             // most 32-key tiles of one attention workgroup
+  int n_split;               // most key segments of a query row
   int from_cache;            // 1: the chunk's keys are cache rows too (verify)
   float scale_log2;
 };
 struct PrefillGeom {
-  int n_pad, h_pad, n_split;
+  int n_pad, h_pad;
+  int max_split;             // key segments per query row that the partial area holds
   size_t kx_off, vt_off, ml_off, o_off, total;
 };
 PrefillGeom prefill_geom(int num_q, int num_kv, int n_tok, int start_pos);
-hipError_t launch_prefill_tq3(const PrefillArgs& a, int gqa, const uint16_t* q, const uint16_t* k,
+// Token groups and key segments of a call (a.hist, h_pad, n_pad, from_cache set)
+// into a.tok_groups, a.seg_tiles, a.n_split <= max_split.
+void prefill_schedule(PrefillArgs& a, int max_split);
+hipError_t launch_prefill_tq3(const PrefillArgs& a, int max_split, int gqa, const uint16_t* q, const uint16_t* k,
                               const uint16_t* v, uint16_t* out, hipStream_t stream);
 
 }  // namespace qkv

@@ -59,6 +59,7 @@ struct AttnArgs {
   // -1 after the last); split z takes entries z * ceil(top_k / k_splits) ..
   const int32_t* block_index;
   int top_k;
+  int wg_splits;            // splits per workgroup: 1, 2, 4 or 8
   // split API partials (reference layout)
   float* part_m;
   float* part_l;

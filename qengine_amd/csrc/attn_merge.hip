@@ -19,15 +19,36 @@ __global__ __launch_bounds__(256) void split_merge_kernel(const float* __restric
                                                           int sub_n_max, int k_splits) {
   const int qh = blockIdx.x, t = blockIdx.y, d = threadIdx.x;
   const long base = ((long)qh * sub_n_max + t) * k_splits;
+  // Splits eight at a time, the loads of a round all issued before the first is used
+  // (past the last split they repeat it and are not counted), the first round's ahead
+  // of the maximum: up to 8 splits are one memory round trip, not one per split.
+  float ms[8], ls[8], os[8];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const long at = base + min(s0 + i, k_splits - 1);
+      ms[i] = pm[at];
+      ls[i] = pl[at];
+      os[i] = po[at * 256 + d];
+    }
+  };
+  load(0);
   float M = -INFINITY;
-  for (int s = 0; s < k_splits; s++) M = fmaxf(M, pm[base + s]);
+#pragma unroll
+  for (int i = 0; i < 8; i++) M = fmaxf(M, ms[i]);
+  for (int s0 = 8; s0 < k_splits; s0 += 8)
+#pragma unroll
+    for (int i = 0; i < 8; i++) M = fmaxf(M, pm[base + min(s0 + i, k_splits - 1)]);
   float L = 0.f, o = 0.f;
-  for (int s = 0; s < k_splits; s++) {
-    const float ms = pm[base + s], ls = pl[base + s];
-    if (!__builtin_isfinite(ms) || ls <= 0.0f) continue;
-    const float w = __expf(ms - M);
-    L += w * ls;
-    o += w * po[(base + s) * 256 + d];
+  for (int s0 = 0; s0 < k_splits; s0 += 8) {
+    if (s0) load(s0);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      if (s0 + i >= k_splits || !__builtin_isfinite(ms[i]) || ls[i] <= 0.0f) continue;
+      const float w = __expf(ms[i] - M);
+      L += w * ls[i];
+      o += w * os[i];
+    }
   }
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   out[((long)t * num_q + qh) * 256 + d] = (uint16_t)f2h(o * inv);

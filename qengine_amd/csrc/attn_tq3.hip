@@ -258,11 +258,10 @@ struct TileRegs {
 
 // prow: cache row of the tile's first key (64 consecutive rows, wave-uniform);
 // the buffer resources are rebased at that row (64-bit byte offset)
-__device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, int h, int lane,
-                                          int row, int col, TileRegs& tr) {
+__device__ __forceinline__ void load_tile_keys(const AttnArgs& p, int prow, int nkv, int h, int row, int col,
+                                               TileRegs& tr) {
   const uint64_t off0 = (uint64_t)(uint32_t)prow * (uint32_t)nkv * 104u;
   const __amdgpu_buffer_rsrc_t rk = cache_rsrc(p.k, off0, p.kv_bytes);
-  const __amdgpu_buffer_rsrc_t rv = cache_rsrc(p.v, off0, p.kv_bytes);
   // keys first (group by group): the score MFMAs of group g only wait for
   // group g, and values arrive while the scores are computed
 #pragma unroll
@@ -277,10 +276,19 @@ __device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, 
       tr.kn[g][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, krow + 52 * j, 0, 0));
     }
   }
+}
+__device__ __forceinline__ void load_tile_values(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRegs& tr) {
+  const uint64_t off0 = (uint64_t)(uint32_t)prow * (uint32_t)nkv * 104u;
+  const __amdgpu_buffer_rsrc_t rv = cache_rsrc(p.v, off0, p.kv_bytes);
   const uint32_t vrow = (uint32_t)(lane * nkv + h) * 104u;
 #pragma unroll
   for (int i = 0; i < 6; i++) tr.vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, vrow + 16 * i, 0, 0);
   tr.vr6 = __builtin_amdgcn_raw_buffer_load_b64(rv, vrow + 96, 0, 0);
+}
+__device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, int h, int lane, int row, int col,
+                                          TileRegs& tr) {
+  load_tile_keys(p, prow, nkv, h, row, col, tr);
+  load_tile_values(p, prow, nkv, h, lane, tr);
 }
 
 // The encoded new key (4 x 13 dwords at nr) written over the registers of
@@ -325,61 +333,50 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
-// Rotate the merged rows back (o = rs*D*H*o_rot per 128-block).  final: divide
-// by L and store fp16 rows [t][q_head][256]; otherwise store the unnormalised
-// f32 partial of reference split `split` (m in natural-log units).
-__device__ void finish_rows(const uint8_t* lds, const AttnArgs& p, int h, int t, int rows,
-                            bool final, int split, uint16_t* out) {
+// Rotate the merged rows back (o = rs*D*H*o_rot per 128-block) and store the
+// unnormalised f32 partials of the reference splits split0 .. split0 + n - 1 (m in
+// natural-log units): row r of split0 + i is merge row i slot + r, its scalars at
+// i rows + r.
+__device__ void finish_rows(const uint8_t* lds, const AttnArgs& p, int h, int t, int rows, int split0, int n,
+                            int slot) {
   const float* mo = reinterpret_cast<const float*>(lds + kLdsMergeO);
   const float* ml = reinterpret_cast<const float*>(lds + kLdsMergeML);
   const int gqa = p.num_q / p.num_kv;
   const int lane = threadIdx.x & 63;
-  for (int w0 = 0; w0 < rows * 2; w0 += kThreads / 16) {
+  n = min(n, p.k_splits - split0);
+  for (int w0 = 0; w0 < n * rows * 2; w0 += kThreads / 16) {
     const int wht = w0 + (threadIdx.x >> 4);
     const int part = threadIdx.x & 15;
-    const int r = wht >> 1, blk = wht & 1;
-    const bool live = wht < rows * 2;
-    const float L = live ? ml[kMlL + r] : 0.f;
-    // the centroid table is scaled by kCenScale: undo it here (fp32)
-    const float scale = (final ? (L > 0.f ? 1.0f / L : 0.f) : 1.0f) * kCenScaleInv;
+    const int ri = wht >> 1, blk = wht & 1, i = ri / rows, r = ri - i * rows;
+    const bool live = wht < n * rows * 2;
     float x[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) x[i] = live ? mo[r * kHD + blk * 128 + part * 8 + i] * scale : 0.f;
+    for (int e = 0; e < 8; e++)   // the centroid table is scaled by kCenScale: undo it here (fp32)
+      x[e] = live ? mo[(i * slot + r) * kHD + blk * 128 + part * 8 + e] * kCenScaleInv : 0.f;
     wht8_inreg(x);
     wht_xor_lanes16(x, lane);
     if (!live) continue;
     const float rs = wht_scale();
     const int qh = h * gqa + r % gqa, tq = t + r / gqa;
-    float y[8];
     const uint32_t sbits = sign_word_sel(part >> 2) >> (8 * (part & 3));  // elements part*8..+7
+    const long mlx = ((long)qh * p.sub_n_max + tq) * p.k_splits + split0 + i;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const bool pos = (sbits >> i) & 1u;
-      const float v = x[i] * rs;
-      y[i] = pos ? v : -v;
+    for (int e = 0; e < 8; e++) {
+      const bool pos = (sbits >> e) & 1u;
+      const float v = x[e] * rs;
+      p.part_o[mlx * kHD + blk * 128 + part * 8 + e] = pos ? v : -v;
     }
-    if (final) {
-      uint32_t pk[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) pk[i] = f2h(y[2 * i]) | (f2h(y[2 * i + 1]) << 16);
-      *reinterpret_cast<uint4*>(out + ((long)tq * p.num_q + qh) * kHD + blk * 128 + part * 8) =
-          make_uint4(pk[0], pk[1], pk[2], pk[3]);
-    } else {
-      const long mlx = ((long)qh * p.sub_n_max + tq) * p.k_splits + split;
-#pragma unroll
-      for (int i = 0; i < 8; i++) p.part_o[mlx * kHD + blk * 128 + part * 8 + i] = y[i];
-      if (blk == 0 && part == 0) {
-        const float M = ml[kMlM + r];
-        p.part_m[mlx] = (M == -INFINITY) ? -INFINITY : M * kLn2;
-        p.part_l[mlx] = ml[kMlL + r];
-      }
+    if (blk == 0 && part == 0) {
+      const float M = ml[kMlM + ri];
+      p.part_m[mlx] = (M == -INFINITY) ? -INFINITY : M * kLn2;
+      p.part_l[mlx] = ml[kMlL + ri];
     }
   }
 }
 
 // MODE 0: fast path (final fp16 rows).  MODE 1: reference split partials.
 // MODE 2: block-sparse split partials (attention.cuh:2193-2433): one query
-// per workgroup (qpw = 1), split z over the query's selected 64-key blocks.
+// per workgroup (qpw = 1), wg_splits splits of its selected 64-key blocks.
 // CHAIN (fast path, several queries): 16 / GQA queries per workgroup, every
 // MFMA column a real (query, head); the remainders ride in a chained second
 // score product (see score_group).
@@ -527,11 +524,15 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   // waits for a table read (rows past the table's extent read as 0)
   constexpr int kStep = kWaves * kTile;
   // block-sparse: lane k holds entry k of this split's block list; the list
-  // ends at its first -1 (n_sel entries); wave w takes entries w, w + 8, ...
+  // ends at its first -1 (n_sel entries).  A workgroup serves wg_splits
+  // consecutive splits of its query, kWaves / wg_splits (spw) waves each: wave
+  // sw of a split takes entries sw, sw + spw, ...  (a split past the last has
+  // an empty list)
+  const int spw = MODE == 2 ? kWaves / p.wg_splits : kWaves, sw = wave % spw;
   int sel = -1, n_sel = 0;
   if constexpr (MODE == 2) {
     const int per = (p.top_k + p.k_splits - 1) / p.k_splits;
-    const int tk_lo = chunk * per, tk_n = max(0, min(per, p.top_k - tk_lo));
+    const int tk_lo = (chunk * p.wg_splits + wave / spw) * per, tk_n = max(0, min(per, p.top_k - tk_lo));
     const __amdgpu_buffer_rsrc_t rbi = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<int32_t*>(p.block_index), 0, (uint32_t)(p.num_kv * p.sub_n_max * p.top_k * 4),
         kBufferRsrcWord3);
@@ -544,7 +545,7 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
     n_sel = ends ? (int)__builtin_ctzll(ends) : 64;
     sel = e;
   }
-  const int ts0 = MODE == 2 ? (wave < n_sel ? __builtin_amdgcn_readlane(sel, wave) * kTile : 0)
+  const int ts0 = MODE == 2 ? (sw < n_sel ? __builtin_amdgcn_readlane(sel, sw) * kTile : 0)
                             : lo + wave * kTile;
   const __amdgpu_buffer_rsrc_t rbt = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int32_t*>(p.block_tables), 0,
@@ -736,9 +737,16 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   float* st = reinterpret_cast<float*>(lds + kLdsStage + wave * kStageBytes);
   uint32_t* stu = reinterpret_cast<uint32_t*>(st);
 
+  // The split forms, whose workgroups are few and walk several tiles, load the next
+  // tile's keys ahead (18,016 keys in 8 splits, GQA 6: 33.0 -> 29.4 us with the merge).
+  // The fast path has one tile per wave at most contexts and two waves per SIMD to
+  // overlap at the others: nothing at 131,072 keys, and paged slots lose (102 -> 109 us).
+  constexpr bool kPrefetch = MODE >= 1;
+  int next_row = 0;   // cache row of the wave's next tile, whose keys are on their way
   // One 64-key tile.  The wave's first tile is a separate instance: its loads
   // were issued with the setup, and its accumulators start at zero.
-  auto tile_body = [&](auto first_tag, int ts) {
+  // next: first key of the wave's next tile, < 0 if this is its last.
+  auto tile_body = [&](auto first_tag, int ts, int next) {
     constexpr bool first = decltype(first_tag)::value;
     auto& kq = tr.kq;
     auto& kn = tr.kn;
@@ -787,6 +795,12 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // the key registers are free: the next tile's keys fly during the softmax and the
+    // value products (its values, during its scores: there are no registers for both)
+    if (kPrefetch && next >= 0) {
+      next_row = wave_tile_row(next);
+      load_tile_keys(p, next_row, p.num_kv, h, row, col, tr);
+    }
 
     // dense is wave-uniform: the common full tile (every key visible to every
     // query of the group) skips the per-key rule
@@ -868,26 +882,33 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   // lo and hi are wave-uniform (a paged workgroup serves one query): the tile
   // loop is a scalar loop
   if constexpr (MODE == 2) {
-    if (wave < n_sel) {
-      tile_body(std::true_type{}, ts0);
-      for (int k = wave + kWaves; k < n_sel; k += kWaves) {
-        const int ts = __builtin_amdgcn_readlane(sel, k) * kTile;
-        load_tile(p, ts, p.num_kv, h, lane, row, col, tr);
-        tile_body(std::false_type{}, ts);
+    auto tile = [&](int k) { return k < n_sel ? __builtin_amdgcn_readlane(sel, k) * kTile : -1; };
+    if (sw < n_sel) {
+      int ts = tile(sw + spw);
+      tile_body(std::true_type{}, ts0, ts);
+      for (int k = sw + spw; k < n_sel; k += spw) {
+        const int next = tile(k + spw);
+        load_tile_values(p, next_row, p.num_kv, h, lane, tr);
+        tile_body(std::false_type{}, ts, next);
+        ts = next;
       }
     } else {
 #pragma unroll
       for (int t = 0; t < 16; t++) acc[t] = f4_t{0.f, 0.f, 0.f, 0.f};
     }
   } else if (ts0 < hi) {
+    auto following = [&](int ts) { return ts + kStep < hi ? ts + kStep : -1; };
     if (APPEND && fa_wave == wave && ts0 <= p.start_pos && p.start_pos < ts0 + kTile)
       patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts0, lane, row, col);
-    tile_body(std::true_type{}, ts0);
+    tile_body(std::true_type{}, ts0, following(ts0));
     for (int ts = ts0 + kStep; ts < hi; ts += kStep) {
-      load_tile(p, wave_tile_row(ts), p.num_kv, h, lane, row, col, tr);
+      if constexpr (kPrefetch)
+        load_tile_values(p, next_row, p.num_kv, h, lane, tr);
+      else
+        load_tile(p, wave_tile_row(ts), p.num_kv, h, lane, row, col, tr);
       if (APPEND && fa_wave == wave && ts <= p.start_pos && p.start_pos < ts + kTile)
         patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts, lane, row, col);
-      tile_body(std::false_type{}, ts);
+      tile_body(std::false_type{}, ts, following(ts));
     }
   } else {
 #pragma unroll
@@ -931,6 +952,30 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   // in a register through the tile loop)
   int gqa_m = gqa;
   asm volatile("" : "+s"(gqa_m));
+  if constexpr (MODE == 2) {
+    // rows of split i, waves i spw ..: merged into slot (i spw, row), scalars at i rows + row
+    for (int idx = threadIdx.x; idx < p.wg_splits * rows * 64; idx += kThreads) {
+      const int ri = idx >> 6, d4 = (idx & 63) * 4, r = ri % rows, w0 = ri / rows * spw;
+      float M = -INFINITY;
+      for (int w = w0; w < w0 + spw; w++) M = fmaxf(M, ml[kMlW0 + w * 16 + r]);
+      float L = 0.f;
+      f4_t o = {0.f, 0.f, 0.f, 0.f};
+      for (int w = w0; w < w0 + spw; w++) {
+        const float mw = ml[kMlW0 + w * 16 + r];
+        const float wt = (mw == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
+        L += wt * ml[kMlLw0 + w * 16 + r];
+        o += wt * *reinterpret_cast<const f4_t*>(mo + (w * 16 + r) * kHD + d4);
+      }
+      *reinterpret_cast<f4_t*>(mo + (w0 * 16 + r) * kHD + d4) = o;   // own elements only
+      if (d4 == 0) {
+        ml[kMlM + ri] = M;
+        ml[kMlL + ri] = L;
+      }
+    }
+    __syncthreads();
+    finish_rows(lds, p, h, t0, rows, chunk * p.wg_splits, p.wg_splits, 16 * spw);
+    return;
+  }
   for (int idx = threadIdx.x; idx < rows * 64; idx += kThreads) {
     const int r = idx >> 6, d4 = (idx & 63) * 4;
     float M = -INFINITY;
@@ -945,7 +990,7 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
       L += wt * ml[kMlLw0 + w * 16 + r];
       o += wt * *reinterpret_cast<const f4_t*>(mo + (w * 16 + r) * kHD + d4);
     }
-    if constexpr (MODE >= 1) {
+    if constexpr (MODE == 1) {
       *reinterpret_cast<f4_t*>(mo + r * kHD + d4) = o;   // wave-0 slot, own elements only
       if (d4 == 0) {
         ml[kMlM + r] = M;
@@ -956,9 +1001,9 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
     }
   }
 
-  if constexpr (MODE >= 1) {
+  if constexpr (MODE == 1) {
     __syncthreads();
-    finish_rows(lds, p, h, t0, rows, false, chunk, nullptr);
+    finish_rows(lds, p, h, t0, rows, chunk, 1, 0);
     return;
   }
 

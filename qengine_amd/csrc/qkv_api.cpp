@@ -397,6 +397,19 @@ int qkv_block_index_ms(const uint16_t* q, const uint16_t* k_pool, const uint16_t
   return launch_status(qkv::launch_block_index(a, static_cast<float*>(workspace), stream));
 }
 
+// Splits served by one workgroup of the block-sparse attention.  Its 8 waves take a
+// 64-key block each, so a split of fewer blocks leaves waves idle; and one workgroup
+// fits a CU, so more than 256 run in rounds that each pay the setup and the merge.
+// Twice the splits per workgroup while either holds and its rows fit the 16 merge rows
+// (16 queries, 8 splits of 8 blocks, 4 kv heads: 28 -> 22 us).
+static int sparse_wg_splits(int gqa, int units, int top_k, int k_splits) {
+  int s = 1;
+  const int per = (top_k + k_splits - 1) / k_splits;   // blocks of a split
+  while (s < 8 && s < k_splits && 2 * s * gqa <= 16 && (2 * s * per <= 8 || (long)units * ((k_splits + s - 1) / s) > 256))
+    s *= 2;
+  return s;
+}
+
 int qkv_attn_block_sparse_split_tq3(const uint16_t* q, const qkv_block_tq3* k,
                                     const qkv_block_tq3* v, const int32_t* block_index,
                                     float* part_m, float* part_l, float* part_o, int num_q,
@@ -425,7 +438,8 @@ int qkv_attn_block_sparse_split_tq3(const uint16_t* q, const qkv_block_tq3* k,
   a.kv_bytes = (uint64_t)(start_pos + sub_n) * num_kv * 104;
   a.active_end_max = start_pos + sub_n;
   a.k_splits = k_splits;
-  a.n_chunks = k_splits;
+  a.wg_splits = sparse_wg_splits(num_q / num_kv, num_kv * sub_n, top_k, k_splits);
+  a.n_chunks = (k_splits + a.wg_splits - 1) / a.wg_splits;
   a.scale_log2 = scale * qkv::kLog2e;
   a.tree_mask = tree_mask;
   a.block_index = block_index;

@@ -87,105 +87,127 @@ __global__ __launch_bounds__(kSpThreads) void tq3_kpool_kernel(KpoolArgs a) {
 }
 
 constexpr int kScBlocks = 32;          // blocks scored per workgroup
-constexpr int kScQueries = 8;          // queries scored per workgroup
-constexpr int kScPitchDw = 129;        // staged pool row: 128 dwords + 1 (conflict-free lanes)
+constexpr int kScPitchDw = 132;        // staged pool row: 128 dwords + 4 (16-byte reads of 16 rows: 64 banks)
+typedef uint32_t u4a4_t __attribute__((ext_vector_type(4), aligned(4)));
 
-// Block scores, one workgroup per (kv head, 32 blocks, 8 queries).  The
+// One pair of dimensions: s + (q0 m0 + q1 m1), both products exact in fp32, their
+// sum rounded once (an FMA onto the other product), then added to s.  The operands
+// are fp16 halves (v_fma_mix_f32; q1 m1 + 0 is exact).  (v_dot2_f32_f16 does not
+// give that rounding.)
+__device__ __forceinline__ float pair_add(float s, uint32_t q, uint32_t m) {
+  const float hi = __builtin_fmaf(h2f(q >> 16), h2f(m >> 16), 0.0f);
+  return s + __builtin_fmaf(h2f(q & 0xffffu), h2f(m & 0xffffu), hi);
+}
+
+// Block scores, one workgroup per (kv head, 32 blocks, 8 NQ queries).  The
 // blocks' mean and max-abs rows are staged in LDS; the GQA-mean queries
 // (fp16-rounded, as the reference forms them, sparse_index.cuh:243-252) sit in
-// LDS as fp16 pairs; thread (t, b) runs block b's two dot products for query
-// t over the 128 pairs in the reference's order: each pair's products are
-// exact and their sum is rounded once (an FMA onto the other exact product),
-// then added to the running fp32 sum.  (v_dot2_f32_f16 does not give that
-// rounding.)  Scores (-inf past the
-// query's causal block) go to the workspace [num_kv][sub_n][n_blocks].
+// LDS as fp16 pairs; thread (t, b) runs block b's two dot products for queries
+// t, t + 8 .. over the 128 pairs in the reference's order (pair_add).  Scores (-inf
+// past the query's causal block) go to the workspace [num_kv][sub_n][n_blocks].
+// Half the VALU's 3 operations per pair and product, half the latency of the inputs:
+// 16 queries over 2,049 blocks, 14.3 -> 11.3 us (with converted operands and a
+// 4-byte LDS read each before).  NQ = 2 (more than 8 queries) reads every staged row
+// once for two queries.
+template <int NQ>
 __global__ __launch_bounds__(kSpThreads) void block_score_kernel(BlockIndexArgs a, float* scores) {
-  __shared__ uint32_t rows_mean[kScBlocks * kScPitchDw];
-  __shared__ uint32_t rows_max[kScBlocks * kScPitchDw];
-  __shared__ uint32_t qa2[kScQueries * kSpHD / 2];   // fp16 pairs
+  constexpr int kQueries = 8 * NQ;
+  __shared__ __attribute__((aligned(16))) uint32_t rows_mean[kScBlocks * kScPitchDw];
+  __shared__ __attribute__((aligned(16))) uint32_t rows_max[kScBlocks * kScPitchDw];
+  __shared__ __attribute__((aligned(16))) uint32_t qa2[kQueries * kSpHD / 2];   // fp16 pairs
   const int nb_wg = (a.n_blocks + kScBlocks - 1) / kScBlocks;
-  const int nq_wg = (a.sub_n + kScQueries - 1) / kScQueries;
+  const int nq_wg = (a.sub_n + kQueries - 1) / kQueries;
   const int qg = blockIdx.x % nq_wg, r = blockIdx.x / nq_wg;
-  const int h = r / nb_wg, b0 = (r - h * nb_wg) * kScBlocks, t0 = qg * kScQueries;
-  const int nt = min(kScQueries, a.sub_n - t0);
+  const int h = r / nb_wg, b0 = (r - h * nb_wg) * kScBlocks, t0 = qg * kQueries;
+  const int nt = min(kQueries, a.sub_n - t0);
   const int tid = threadIdx.x;
   const int gqa = a.num_q / a.num_kv;
-  // Every load of the staging and of the query is issued before the first
-  // one is used (one memory round trip for the workgroup's inputs).
+  // Every load of the query and of the staging is issued before the first one is
+  // used (one memory round trip for the workgroup's inputs).  GQA-mean queries:
+  // thread i forms 8 dims of query i / 32 from its 8 (or gqa) heads' 16-byte
+  // pieces (heads past gqa re-read the last head and are not added; queries past
+  // the last re-read the last)
+  u4a4_t qv[NQ][8];
+#pragma unroll
+  for (int k = 0; k < NQ; k++) {
+    const int tq = min((tid >> 5) + 8 * k, nt - 1);
+#pragma unroll
+    for (int g = 0; g < 8; g++)
+      qv[k][g] = *reinterpret_cast<const u4a4_t*>(
+          a.q + ((long)(t0 + tq) * a.num_q + h * gqa + min(g, gqa - 1)) * kSpHD + (tid & 31) * 8);
+  }
   // 32 blocks x {mean, max} x 512 B: 2048 16-byte pieces, 8 per thread
-  // (blocks past the pool's end are read at its last block and zeroed)
+  // (blocks past the pool's end are read at its last block and not stored)
   static_assert(kScBlocks * 64 == 8 * kSpThreads, "8 staging pieces per thread");
-  uint4 pv[8];
+  u4_t pv[8];
 #pragma unroll
   for (int k = 0; k < 8; k++) {
     const int piece = tid + k * kSpThreads;
     const int b = piece >> 6, w = piece & 63;   // w < 32: mean, else max; 8 dims each
     const int nbk = min(b0 + b, a.n_blocks - 1);
-    pv[k] = *reinterpret_cast<const uint4*>((w < 32 ? a.k_pool : a.k_pool_max) +
-                                            ((long)h * a.stride + nbk) * kSpHD + (w & 31) * 8);
+    pv[k] = *reinterpret_cast<const u4_t*>((w < 32 ? a.k_pool : a.k_pool_max) +
+                                           ((long)h * a.stride + nbk) * kSpHD + (w & 31) * 8);
   }
-  // GQA-mean query pairs: thread i < nt * 128 forms pair c of query tq from
-  // the 8 (or gqa) heads' fp16 pairs, loaded together (heads past gqa re-read
-  // the last head and are not added)
-  static_assert(kScQueries * kSpHD / 2 == 4 * kSpThreads, "4 query pairs per thread");
-  uint32_t qv[4][8];
+  const float inv_g = a.inv_gqa;
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int i = min(tid + k * kSpThreads, nt * kSpHD / 2 - 1);
-    const int tq = i / (kSpHD / 2), c = 2 * (i - tq * (kSpHD / 2));
+  for (int k = 0; k < NQ; k++) {
+    float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};   // heads in order (the reference's sum)
 #pragma unroll
-    for (int g = 0; g < 8; g++)
-      qv[k][g] = *reinterpret_cast<const uint32_t*>(
-          a.q + ((long)(t0 + tq) * a.num_q + h * gqa + min(g, gqa - 1)) * kSpHD + c);
+    for (int g = 0; g < 8; g++) {
+      const uint32_t keep = g < gqa ? 0xffffffffu : 0u;   // (+ 0 leaves the sum as it is)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        s[2 * e] += h2f(qv[k][g][e] & keep & 0xffffu);
+        s[2 * e + 1] += h2f((qv[k][g][e] & keep) >> 16);
+      }
+    }
+    uint32_t pk[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      // the reference rounds s * (1/GQA) to fp32, then to fp16: the empty asm
+      // keeps the fp32 product (no fused fp16-rounding mixed FMA)
+      float p0 = s[2 * e] * inv_g, p1 = s[2 * e + 1] * inv_g;
+      asm volatile("" : "+v"(p0), "+v"(p1));
+      pk[e] = f2h(p0) | (f2h(p1) << 16);
+    }
+    *reinterpret_cast<uint4*>(qa2 + (8 * k + (tid >> 5)) * (kSpHD / 2) + (tid & 31) * 4) =
+        make_uint4(pk[0], pk[1], pk[2], pk[3]);
   }
 #pragma unroll
   for (int k = 0; k < 8; k++) {
     const int piece = tid + k * kSpThreads;
     const int b = piece >> 6, w = piece & 63;
-    const uint4 v = b0 + b < a.n_blocks ? pv[k] : make_uint4(0u, 0u, 0u, 0u);
-    uint32_t* d = (w < 32 ? rows_mean : rows_max) + b * kScPitchDw + (w & 31) * 4;
-    d[0] = v.x;
-    d[1] = v.y;
-    d[2] = v.z;
-    d[3] = v.w;
-  }
-  const float inv_g = a.inv_gqa;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int i = tid + k * kSpThreads;
-    if (i < nt * kSpHD / 2) {
-      float s0 = 0.0f, s1 = 0.0f;   // heads in order (the reference's sum)
-#pragma unroll
-      for (int g = 0; g < 8; g++)
-        if (g < gqa) {
-          s0 += h2f(qv[k][g] & 0xffffu);
-          s1 += h2f(qv[k][g] >> 16);
-        }
-      // the reference rounds s * (1/GQA) to fp32, then to fp16: the empty asm
-      // keeps the fp32 product (no fused fp16-rounding mixed FMA)
-      float p0 = s0 * inv_g, p1 = s1 * inv_g;
-      asm volatile("" : "+v"(p0), "+v"(p1));
-      qa2[i] = f2h(p0) | (f2h(p1) << 16);
-    }
+    *reinterpret_cast<u4_t*>((w < 32 ? rows_mean : rows_max) + b * kScPitchDw + (w & 31) * 4) = pv[k];
   }
   __syncthreads();
   // thread -> (query tq, block b): 32 lanes of a wave are the 32 blocks of one query
   const int tq = tid / kScBlocks, b = tid - tq * kScBlocks;
-  if (tq < nt) {
-    const uint32_t* mn = rows_mean + b * kScPitchDw;
-    const uint32_t* mx = rows_max + b * kScPitchDw;
-    const uint32_t* q = qa2 + tq * (kSpHD / 2);
-    float s_mean = 0.0f, s_max = 0.0f;
-#pragma unroll 16
-    for (int c2 = 0; c2 < kSpHD / 2; c2++) {
-      const uint32_t qw = q[c2], m2 = mn[c2], x2 = mx[c2];
-      const float q0 = h2f(qw & 0xffffu), q1 = h2f(qw >> 16);
-      s_mean += __builtin_fmaf(q0, h2f(m2 & 0xffffu), q1 * h2f(m2 >> 16));
-      s_max += __builtin_fmaf(q0, h2f(x2 & 0xffffu), q1 * h2f(x2 >> 16));
+  const uint32_t* mn = rows_mean + b * kScPitchDw;
+  const uint32_t* mx = rows_max + b * kScPitchDw;
+  const uint32_t* q = qa2 + tq * (kSpHD / 2);
+  float s_mean[NQ], s_max[NQ];
+#pragma unroll
+  for (int k = 0; k < NQ; k++) s_mean[k] = s_max[k] = 0.0f;
+#pragma unroll 4
+  for (int c = 0; c < kSpHD / 2; c += 4) {
+    const uint4 m4 = *reinterpret_cast<const uint4*>(mn + c), x4 = *reinterpret_cast<const uint4*>(mx + c);
+    const uint32_t m[4] = {m4.x, m4.y, m4.z, m4.w}, x[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+    for (int k = 0; k < NQ; k++) {
+      const uint4 q4 = *reinterpret_cast<const uint4*>(q + 8 * k * (kSpHD / 2) + c);
+      const uint32_t qw[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        s_mean[k] = pair_add(s_mean[k], qw[e], m[e]);
+        s_max[k] = pair_add(s_max[k], qw[e], x[e]);
+      }
     }
-    const int n = b0 + b, t = t0 + tq;
-    if (n < a.n_blocks) {
-      const float sc = fmaxf(s_mean, a.beta * s_max);
+  }
+#pragma unroll
+  for (int k = 0; k < NQ; k++) {
+    const int n = b0 + b, t = t0 + tq + 8 * k;
+    if (n < a.n_blocks && tq + 8 * k < nt) {
+      const float sc = fmaxf(s_mean[k], a.beta * s_max[k]);
       scores[((long)h * a.sub_n + t) * a.n_blocks + n] = n > (a.start_pos + t) / a.bsn ? -INFINITY : sc;
     }
   }
@@ -199,131 +221,135 @@ __global__ __launch_bounds__(kSpThreads) void block_score_kernel(BlockIndexArgs 
 // of the score (-0 and +0 equal):
 //   1. four 8-bit passes narrow the key T of the top_k-th pick (a 256-bin
 //      histogram of the keys that share the digits found so far, and a
-//      suffix scan over the bins);
+//      suffix scan over the bins, by every wave for itself);
 //   2. the picks are the blocks with key > T and the lowest-numbered `need`
-//      blocks with key == T (a block-wide scan in block order);
-//   3. a second scan gives each pick its place in the ascending list.
-// Each thread owns a contiguous run of blocks.
-constexpr int kTkThreads = 256;
+//      blocks with key == T;
+//   3. their places in the ascending list follow from the counts of the waves
+//      before and ballots within the wave.
+// A chain of latencies, not of work: the keys stay in registers (wave w holds
+// blocks 64 KPT w ..; slot j of lane l is block 64 (KPT w + j) + l) and there are
+// six barriers.  2,049 blocks, 64 rows: 5 us (256 threads with the keys in LDS
+// and a scan through LDS in every pass: 14).
+constexpr int kTkWaves = 16, kTkThreads = 64 * kTkWaves;
 
 __device__ __forceinline__ uint32_t order_key(float v) {
   const uint32_t b = __float_as_uint(v == 0.0f ? 0.0f : v);
   return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 __device__ __forceinline__ bool pickable(float v) { return v > -INFINITY; }   // false for NaN
+// key of a pickable score, 0 otherwise (every pickable score, > -inf and not
+// NaN, has a key above 0x007FFFFF)
+__device__ __forceinline__ uint32_t select_key(float v) { return pickable(v) ? order_key(v) : 0u; }
 
-// Exclusive scan of v over the workgroup (block order = thread order), and the total.
-__device__ __forceinline__ int block_scan(int v, int* wtot, int& total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int inc = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int u = __shfl_up(inc, d, 64);
-    if (lane >= d) inc += u;
-  }
-  if (lane == 63) wtot[wave] = inc;
-  __syncthreads();
-  int off = 0, tot = 0;
-#pragma unroll
-  for (int w = 0; w < kTkThreads / 64; w++) {
-    const int x = wtot[w];
-    off += w < wave ? x : 0;
-    tot += x;
-  }
-  __syncthreads();
-  total = tot;
-  return off + inc - v;
+template <int CTRL, int MASK>
+__device__ __forceinline__ int dpp_add(int v) {   // v + the lane CTRL names (0 if none)
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, MASK, 0xf, false);
+}
+__device__ __forceinline__ int wave_scan(int v) {   // inclusive
+  v = dpp_add<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);   // row_bcast:15, :31
+  return dpp_add<0x143, 0xc>(v);
+}
+__device__ __forceinline__ int lanes_below(uint64_t mask) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// Rows of up to kSelLdsKeys blocks are read once and keep their keys in LDS
-// for all passes; longer rows read the scores from the workspace in every pass.
-constexpr int kSelLdsKeys = 8192;
+// KPT: keys per thread.  KPT 0: any number of blocks, the keys read from the
+// workspace in every pass.
+template <int KPT>
 __global__ __launch_bounds__(kTkThreads) void block_select_kernel(BlockIndexArgs a, const float* scores) {
-  __shared__ uint32_t keys_s[kSelLdsKeys];
-  __shared__ int hist[256];
-  __shared__ int wtot[kTkThreads / 64];
-  __shared__ int found[2];
+  __shared__ __attribute__((aligned(16))) int hist[4][256];
+  __shared__ int wcnt[2][kTkWaves];
   const int h = blockIdx.x % a.num_kv, t = blockIdx.x / a.num_kv;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const float* src = scores + ((long)h * a.sub_n + t) * a.n_blocks;
   int32_t* row = a.block_index + ((long)h * a.sub_n_max + t) * a.top_k;
-  const int per = (a.n_blocks + kTkThreads - 1) / kTkThreads;
-  const int i0 = min(tid * per, a.n_blocks), i1 = min(i0 + per, a.n_blocks);
-  // key of block i: the order key of a pickable score, 0 otherwise (every
-  // pickable score, > -inf and not NaN, has a key above 0x007FFFFF)
-  const bool staged = a.n_blocks <= kSelLdsKeys;
-  auto key_from = [](float v) -> uint32_t { return pickable(v) ? order_key(v) : 0u; };
-  if (staged) {
-    for (int i = tid; i < a.n_blocks; i += kTkThreads) keys_s[i] = key_from(src[i]);
+  const int kpt = KPT ? KPT : (a.n_blocks + kTkThreads - 1) / kTkThreads;   // slots per thread
+  const int base = 64 * kpt * wave + lane;
+  uint32_t key[KPT ? KPT : 1];
+  if constexpr (KPT) {
+    float v[KPT];
+#pragma unroll
+    for (int j = 0; j < KPT; j++) v[j] = src[min(base + 64 * j, a.n_blocks - 1)];
+#pragma unroll
+    for (int j = 0; j < KPT; j++) key[j] = base + 64 * j < a.n_blocks ? select_key(v[j]) : 0u;
+  }
+  auto each = [&](auto f) {   // f(slot, key): every lane of the wave, slots in order
+    if constexpr (KPT) {
+#pragma unroll
+      for (int j = 0; j < KPT; j++) f(j, key[j]);
+    } else {
+      for (int j = 0; j < kpt; j++) f(j, base + 64 * j < a.n_blocks ? select_key(src[base + 64 * j]) : 0u);
+    }
+  };
+  static_assert(kTkThreads == 4 * 256, "one thread per bin of the four histograms");
+  reinterpret_cast<int*>(hist)[tid] = 0;
+  __syncthreads();
+  uint32_t T = 0u, mask = 0u;   // the digits of the top_k-th pick's key found so far
+  int need = a.top_k;           // its rank among the keys that share them
+  bool all = false;             // no more pickable blocks than picks: every one is picked
+#pragma unroll
+  for (int pass = 0; pass < 4; pass++) {
+    const int shift = 24 - 8 * pass;
+    if (!all) {
+      each([&](int, uint32_t k) {
+        if (k != 0u && (k & mask) == T) atomicAdd(&hist[pass][(k >> shift) & 255u], 1);
+      });
+    }
     __syncthreads();
-  }
-  auto key_at = [&](int i) -> uint32_t { return staged ? keys_s[i] : key_from(src[i]); };
-
-  int n_ok = 0;
-  for (int i = i0; i < i1; i++) n_ok += key_at(i) != 0u;
-  int total;
-  (void)block_scan(n_ok, wtot, total);
-  const bool all = total <= a.top_k;   // every pickable block is picked
-  uint32_t T = 0u;
-  int need = 0;
-  if (!all) {
-    uint32_t prefix = 0u, mask = 0u;
-    int kk = a.top_k;   // rank of the pick sought among the keys sharing `prefix`
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      hist[tid] = 0;
-      __syncthreads();
-      for (int i = i0; i < i1; i++) {
-        const uint32_t key = key_at(i);
-        if (key != 0u && (key & mask) == prefix) atomicAdd(&hist[(key >> shift) & 255u], 1);
+    if (!all) {
+      // lane l: bins 255 - 4 l .. 252 - 4 l
+      const int4 c = *reinterpret_cast<const int4*>(&hist[pass][252 - 4 * lane]);
+      const int sum = (c.x + c.y) + (c.z + c.w), upto = wave_scan(sum);
+      if (pass == 0 && __builtin_amdgcn_readlane(upto, 63) <= a.top_k) {
+        all = true;
+      } else {
+        // the lane whose bins reach the rank: the first whose running count does
+        const int l = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= need));
+        int left = need - __builtin_amdgcn_readlane(upto - sum, l), digit = 255 - 4 * l;
+        const int cnt[4] = {__builtin_amdgcn_readlane(c.w, l), __builtin_amdgcn_readlane(c.z, l),
+                            __builtin_amdgcn_readlane(c.y, l), __builtin_amdgcn_readlane(c.x, l)};
+        bool there = false;
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+          there = there || left <= cnt[e];
+          left -= there ? 0 : cnt[e];
+          digit -= there ? 0 : 1;
+        }
+        T |= (uint32_t)digit << shift;
+        mask |= 255u << shift;
+        need = left;
       }
-      __syncthreads();
-      // suffix sums: thread tid takes bin 255 - tid
-      const int c = hist[255 - tid];
-      int tot;
-      const int above = block_scan(c, wtot, tot);   // keys in bins above 255 - tid
-      if (above < kk && above + c >= kk) {
-        found[0] = 255 - tid;
-        found[1] = kk - above;
-      }
-      __syncthreads();
-      prefix |= (uint32_t)found[0] << shift;
-      mask |= 255u << shift;
-      kk = found[1];
-      __syncthreads();
-    }
-    T = prefix;
-    need = kk;   // picks among the blocks whose key is exactly T
-  }
-  // picks, in block order
-  int n_eq = 0;
-  if (!all)
-    for (int i = i0; i < i1; i++) n_eq += key_at(i) == T;
-  int tot_eq;
-  int eq_rank = block_scan(n_eq, wtot, tot_eq);
-  int n_pick = 0;
-  for (int i = i0; i < i1; i++) {
-    const uint32_t key = key_at(i);
-    if (key == 0u) continue;
-    if (all || key > T) {
-      n_pick++;
-    } else if (key == T) {
-      n_pick += eq_rank < need;
-      eq_rank++;
     }
   }
-  int n_total;
-  int pos = block_scan(n_pick, wtot, n_total);
-  eq_rank -= n_eq;   // back to this thread's first equal key
-  for (int i = i0; i < i1; i++) {
-    const uint32_t key = key_at(i);
-    if (key == 0u) continue;
-    bool pick = all || key > T;
-    if (!all && key == T) {
-      pick = eq_rank < need;
-      eq_rank++;
-    }
-    if (pick) row[pos++] = i;
+  // picks: keys above T, and the first `need` of those equal to it, in block order
+  auto above = [&](uint32_t k) { return all ? k != 0u : k > T; };
+  auto equal = [&](uint32_t k) { return !all && k == T; };
+  int n_gt = 0, n_eq = 0;
+  each([&](int, uint32_t k) {
+    n_gt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(above(k)));
+    n_eq += __builtin_popcountll(__builtin_amdgcn_ballot_w64(equal(k)));
+  });
+  if (lane == 0) {
+    wcnt[0][wave] = n_gt;
+    wcnt[1][wave] = n_eq;
   }
+  __syncthreads();
+  const int sg = wave_scan(lane < kTkWaves ? wcnt[0][lane & (kTkWaves - 1)] : 0);
+  const int se = wave_scan(lane < kTkWaves ? wcnt[1][lane & (kTkWaves - 1)] : 0);
+  int gt = __builtin_amdgcn_readlane(sg, wave) - n_gt, eq = __builtin_amdgcn_readlane(se, wave) - n_eq;
+  each([&](int j, uint32_t k) {
+    const uint64_t mg = __builtin_amdgcn_ballot_w64(above(k)), me = __builtin_amdgcn_ballot_w64(equal(k));
+    const int eq_here = eq + lanes_below(me);   // equal keys of lower blocks
+    if (above(k) || (equal(k) && eq_here < need)) row[gt + lanes_below(mg) + min(eq_here, need)] = base + 64 * j;
+    gt += __builtin_popcountll(mg);
+    eq += __builtin_popcountll(me);
+  });
+  const int n_total = __builtin_amdgcn_readlane(sg, 63) + min(__builtin_amdgcn_readlane(se, 63), need);
   for (int j = n_total + tid; j < a.top_k; j += kTkThreads) row[j] = -1;
 }
 
@@ -336,13 +362,21 @@ hipError_t launch_tq3_kpool(const KpoolArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_block_index(const BlockIndexArgs& a, float* scores, hipStream_t stream) {
-  const int nb_wg = (a.n_blocks + kScBlocks - 1) / kScBlocks;
-  const int nq_wg = (a.sub_n + kScQueries - 1) / kScQueries;
-  if (nb_wg == 0 || nq_wg == 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(block_score_kernel, dim3((unsigned)(a.num_kv * nb_wg * nq_wg)), dim3(kSpThreads), 0,
-                     stream, a, scores);
-  hipLaunchKernelGGL(block_select_kernel, dim3((unsigned)(a.num_kv * a.sub_n)), dim3(kTkThreads), 0,
-                     stream, a, static_cast<const float*>(scores));
+  const bool two = a.sub_n > 8;   // queries per thread
+  const long n_wg = (long)a.num_kv * ((a.n_blocks + kScBlocks - 1) / kScBlocks) * ((a.sub_n + (two ? 15 : 7)) / (two ? 16 : 8));
+  if (n_wg <= 0) return hipErrorInvalidValue;
+  if (two)
+    hipLaunchKernelGGL((block_score_kernel<2>), dim3((unsigned)n_wg), dim3(kSpThreads), 0, stream, a, scores);
+  else
+    hipLaunchKernelGGL((block_score_kernel<1>), dim3((unsigned)n_wg), dim3(kSpThreads), 0, stream, a, scores);
+  const dim3 grid((unsigned)(a.num_kv * a.sub_n)), block(kTkThreads);
+  const float* sc = scores;
+  if (a.n_blocks <= 4 * kTkThreads)
+    hipLaunchKernelGGL((block_select_kernel<4>), grid, block, 0, stream, a, sc);
+  else if (a.n_blocks <= 16 * kTkThreads)
+    hipLaunchKernelGGL((block_select_kernel<16>), grid, block, 0, stream, a, sc);
+  else
+    hipLaunchKernelGGL((block_select_kernel<0>), grid, block, 0, stream, a, sc);
   return hipGetLastError();
 }
 

@@ -99,6 +99,9 @@ struct MqLds {
   static constexpr int kRed = 0;                          // mergers
   static constexpr int kMls = kRed + kWaves * 128 * 4;
   static constexpr int kSum = kMls + 256 * 8;             // [4][64] sums, [64] maxima, [64] record indices
+  static constexpr int kRowPitch = kHD + 4;               // SPLIT: rows to rotate back, kSum's maxima in between
+  static constexpr int kRows = kSum + 10 * 64 * 4;
+  static_assert(kRows + 32 * kRowPitch * 4 <= kEnd, "rows to rotate back (NG = 2)");
   static_assert(kSum + 6 * 64 * 4 <= kP, "end-of-kernel scalars must not reach the probabilities");
   static_assert(!KT || kQlo + 64 * 512 <= kMx, "query scratch must not reach the flags");
   static_assert(kEnd <= 160 * 1024, "LDS");
@@ -271,7 +274,10 @@ __device__ __forceinline__ uint32_t pair_read(const uint8_t* lds, uint32_t w, ui
 }
 
 // NG: 16-column groups of a workgroup, 2 or 4.
-template <bool KT, bool VT, int NG>
+// SPLIT: the split API.  The chunk is a reference split, whose partials (true maximum
+// in natural-log units, sum, unnormalised row in the caller's coordinates) go to
+// part_m / part_l / part_o.
+template <bool KT, bool VT, int NG, bool SPLIT>
 __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARAMS, AttnArgs pin, uint16_t* out) {
   QKV_ATTN_LEAD_APPLY(p, pin);
   static_assert(!KT || VT, "TQ3 keys come with TQ3 values");
@@ -291,6 +297,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     const int g = (r / p.num_kv) * 8 + xcd;
     const int groups = (p.sub_n + p.qpw - 1) / p.qpw;
     has_work = g < groups * p.n_chunks;
+    if (SPLIT && !has_work) return;
     const int tq = has_work ? g / p.n_chunks : 0;
     chunk = has_work ? g - tq * p.n_chunks : 0;
     t0 = tq * p.qpw;
@@ -337,7 +344,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   int lo = 0, hi = 0, hi_first = 0, c_end = 0;
   if (has_work) {
     lo = chunk * p.chunk_keys;
-    c_end = chunk == p.n_chunks - 1 ? active_last : lo + p.chunk_keys;
+    c_end = !SPLIT && chunk == p.n_chunks - 1 ? active_last : lo + p.chunk_keys;
     hi = min(c_end, active_last);
     hi_first = min(c_end, p.start_pos + t0 + 1);
   }
@@ -481,9 +488,11 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   // (a reference that no visible score has touched yet is kNoRef, not -inf: the
   // weights of masked keys are then 0 without a test)
   float m2[kCg], lsum[kCg];
+  float mt[kCg];   // SPLIT: this lane's part of the columns' maxima
 #pragma unroll
   for (int cg = 0; cg < kCg; cg++) {
     m2[cg] = kNoRef;
+    mt[cg] = -INFINITY;
     lsum[cg] = 0.0f;
   }
   f4_t acc[NG][2];
@@ -609,7 +618,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     // (half kg >> 1, kb), stored at unit ^ ((c >> 1) & 7), holds keys
     // 32 (kg >> 1) + 4 kb + 0..3 and + 16..19 (the k order of the value product).
     // Returns the largest score above the reference.
-    float ps[kCg];
+    float ps[kCg], tl[kCg];   // (tl, SPLIT: the columns' maxima above the reference)
     uint8_t* pd = pbuf + c0 * 128 + 16 * (((kg >> 1) * 4 + kb) ^ ((c0 >> 1) & 7)) + 8 * (kg & 1);
     auto put_p = [&](auto DENSE) {
       constexpr bool all = decltype(DENSE)::value;
@@ -633,7 +642,8 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
           d[r] = score(kn, cg, r, m2[cg]);
           if constexpr (!all) d[r] = (vis[cg] >> r & 1u) ? d[r] : -INFINITY;
         }
-        top = fmaxf(top, fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3])));
+        tl[cg] = fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3]));
+        top = fmaxf(top, tl[cg]);
 #pragma unroll
         for (int r = 0; r < 4; r++) pr[r] = __builtin_amdgcn_exp2f(d[r]);
         ps[cg] = (pr[0] + pr[1]) + (pr[2] + pr[3]);
@@ -692,7 +702,9 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       for (int cg = 0; cg < kCg; cg++) {
         const f4_t mk = *reinterpret_cast<const f4_t*>(mx + 4 * (c1 + 16 * cg));
         // (a whole number: every rescale is by an exact power of two)
-        const float mn = fmaxf(m2[cg], __builtin_ceilf(fmaxf(fmaxf(mk[0], mk[1]), fmaxf(mk[2], mk[3]))) - kHead<VT>);
+        const float mm = fmaxf(fmaxf(mk[0], mk[1]), fmaxf(mk[2], mk[3]));
+        const float mn = fmaxf(m2[cg], __builtin_ceilf(mm) - kHead<VT>);
+        if constexpr (SPLIT) mt[cg] = fmaxf(mt[cg], mm);   // (an infinite one shows only here)
         const float corr = __builtin_amdgcn_exp2f(m2[cg] - mn);
         lsum[cg] *= corr;
         m2[cg] = mn;
@@ -718,7 +730,10 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     }
     if (tid == 0) flag_s[b2] = 0;   // (set by tile t + 2, after the next barrier)
 #pragma unroll
-    for (int cg = 0; cg < kCg; cg++) lsum[cg] += ps[cg];
+    for (int cg = 0; cg < kCg; cg++) {
+      lsum[cg] += ps[cg];
+      if constexpr (SPLIT) mt[cg] = fmaxf(mt[cg], tl[cg] + m2[cg]);
+    }
     // ---- values: acc[g][e] += P(16 columns x 32 keys) V(32 keys x 16 dims)
     const uint8_t* pbase = pbuf + (VT ? (wave >> 2) * 64 * 128 : 0);
     auto p_operand = [&](int g, int c2) {   // columns 16 g + n, keys of half c2
@@ -809,7 +824,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   int tid_e = tid;
   asm volatile("" : "+v"(tid_e));
   const int n_e = tid_e & 15, kb_e = (tid_e & 63) >> 4;
-  // ---- records: the waves of a column half hold its sums per key group, every
+  // ---- records (SPLIT: partials): the waves of a column half hold its sums per key group, every
   // wave its dims of every column
   __syncthreads();
   float* sums = reinterpret_cast<float*>(lds + L::kSum);
@@ -826,6 +841,69 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       sums[kg * 64 + c] = l;
       if (kg == 0) sums[4 * 64 + c] = m2[cg];
     }
+    if constexpr (SPLIT) {
+      const float m = xrow_max(mt[cg]);
+      if (kb_e == 0) sums[(6 + kg) * 64 + c] = m;
+    }
+  }
+  if constexpr (SPLIT) {
+    __syncthreads();
+    // rows scaled from the reference to the maximum, and rotated back (TQ3 values)
+    auto column_max = [&](int c) {
+      return fmaxf(fmaxf(sums[6 * 64 + c], sums[7 * 64 + c]), fmaxf(sums[8 * 64 + c], sums[9 * 64 + c]));
+    };
+    auto factor = [&](int c) {
+      const float m = column_max(c);
+      return m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(sums[4 * 64 + c] - m);
+    };
+    auto row_index = [&](int c) {
+      return ((long)(h * gqa_m + c % gqa_m) * p.sub_n_max + t0 + c / gqa_m) * p.k_splits + chunk;
+    };
+    if (tid_e < cols) {
+      const float m = column_max(tid_e), f = factor(tid_e);
+      const long at = row_index(tid_e);
+      p.part_m[at] = m == -INFINITY ? -INFINITY : m * kLn2;
+      p.part_l[at] = f * ((sums[tid_e] + sums[64 + tid_e]) + (sums[128 + tid_e] + sums[192 + tid_e]));
+    }
+    typedef float f2a4_t __attribute__((ext_vector_type(2), aligned(4)));
+    float* rows_s = reinterpret_cast<float*>(lds + L::kRows);
+#pragma unroll
+    for (int g = 0; g < NG; g++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int R = 16 * g + 4 * kb_e + r;
+        if (R >= cols) continue;
+        const float f = factor(R);
+        if constexpr (VT)
+          *reinterpret_cast<f2_t*>(rows_s + R * L::kRowPitch + 32 * wave + 2 * n_e) = f2_t{acc[g][0][r], acc[g][1][r]} * f;
+        else
+          *reinterpret_cast<f2a4_t*>(p.part_o + row_index(R) * kHD + 32 * wave + 2 * n_e) =
+              f2a4_t{acc[g][0][r] * f, acc[g][1][r] * f};
+      }
+    if constexpr (VT) {
+      __syncthreads();
+      const int part = tid_e & 15;
+      const uint32_t sbits = sign_word_sel(part >> 2) >> (8 * (part & 3));   // elements part*8..+7
+      const float rs = wht_scale();
+      for (int u0 = 0; u0 < 2 * cols; u0 += kThreads / 16) {
+        const int u = u0 + (tid_e >> 4), R = u >> 1, blk = u & 1;
+        const bool live = u < 2 * cols;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++)   // the centroid table is scaled by kCenScale: undo it here
+          x[e] = live ? rows_s[R * L::kRowPitch + blk * 128 + part * 8 + e] * kCenScaleInv : 0.0f;
+        wht8_inreg(x);
+        wht_xor_lanes16(x, tid_e & 63);
+        if (!live) continue;
+        float* o = p.part_o + row_index(R) * kHD + blk * 128 + part * 8;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const float v = x[e] * rs;
+          o[e] = ((sbits >> e) & 1u) ? v : -v;
+        }
+      }
+    }
+    return;
   }
   if (tid_e < 64) recs[tid_e] = (int)rec_index(p, h * gqa_m + tid_e % gqa_m, t0 + min(tid_e, cols - 1) / gqa_m, chunk);
   __syncthreads();
@@ -857,9 +935,9 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
 template <bool KT, bool VT>
 static void launch_mq(const AttnArgs& a, int n_wg, uint16_t* out, hipStream_t stream) {
   if (a.qpw * (a.num_q / a.num_kv) > 32)
-    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 4>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 4, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
   else
-    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 2>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 2, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
 }
 
 hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* out, hipStream_t stream) {
@@ -875,6 +953,21 @@ hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* o
     launch_mq<false, true>(a, n_wg, out, stream);
   else
     launch_mq<false, false>(a, n_wg, out, stream);
+  return hipGetLastError();
+}
+
+// The split API's partials (TQ3 caches: at most 32 columns per workgroup).
+hipError_t launch_mq_split(const AttnArgs& a, bool tq3, hipStream_t stream) {
+  const int groups = (a.sub_n + a.qpw - 1) / a.qpw * a.n_chunks;
+  const dim3 grid((groups + 7) / 8 * 8 * a.num_kv), block(kThreads);
+  const bool wide = a.qpw * (a.num_q / a.num_kv) > 32;
+  if (tq3 && wide) return hipErrorInvalidValue;
+  if (tq3)
+    hipLaunchKernelGGL((mq_attn_kernel<true, true, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, nullptr);
+  else if (wide)
+    hipLaunchKernelGGL((mq_attn_kernel<false, false, 4, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, nullptr);
+  else
+    hipLaunchKernelGGL((mq_attn_kernel<false, false, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, nullptr);
   return hipGetLastError();
 }
 

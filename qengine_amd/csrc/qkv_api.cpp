@@ -290,6 +290,51 @@ int check_attn_shape(int num_q, int num_kv, int head_dim, int start_pos, int sub
 
 extern "C" {
 
+// Keys of a reference split (attention.cuh:1944-1951, 2660-2663).
+static int split_keys(int active_end_max, int k_splits) {
+  const int total_tiles = (active_end_max + 31) / 32;
+  return (total_tiles + k_splits - 1) / k_splits * 32;
+}
+
+// Queries per workgroup of at most `columns` (query, head) columns, and the
+// workgroups of all of them.
+struct SplitMq {
+  int queries;
+  long wgs;
+};
+static SplitMq split_mq(int gqa, int num_kv, int sub_n, int k_splits, int columns) {
+  const int most = columns / gqa, groups = (sub_n + most - 1) / most;
+  return {(sub_n + groups - 1) / groups, (long)num_kv * k_splits * groups};
+}
+
+// Whether the split API's call goes to the multi-query kernel: its queries per
+// workgroup, or 0.  A reference split is one workgroup's work however many CUs are
+// idle, so the kernels compare by their rounds of the GPU (one workgroup per CU, TQ3)
+// and by the time of one.  As measured, us over the keys m of a split:
+//   TQ3, 8 / gqa queries per workgroup, a tile per wave   9 + 0.011 m
+//   TQ3, 32 columns per workgroup, tiles one by one      12 + 0.026 m
+// 16 queries in 32 splits, GQA 4: 40.6 -> 15.1 us at 2,048 keys, 55 -> 27 at 18,016,
+// 111 -> 65 at 65,000; in 8 splits (one round either way) 33 at 18,016, not 70.
+static int tq3_split_mq(int gqa, int num_kv, int sub_n, int k_splits, int m) {
+  const int per = 8 / gqa;
+  const long old_wgs = (long)num_kv * k_splits * ((sub_n + per - 1) / per);
+  const SplitMq mq = split_mq(gqa, num_kv, sub_n, k_splits, 32);
+  const long old_rounds = (old_wgs + 255) / 256, rounds = (mq.wgs + 255) / 256;
+  return rounds * (12000 + 26l * m) < old_rounds * (9000 + 11l * m) ? mq.queries : 0;
+}
+// Q8_0: one query per workgroup against every query that 32 columns hold (64 where 32
+// would take several rounds).  One workgroup alone reads its split at the rate of a
+// CU's memory pipe, and so does a pair on one CU together: the multi-query kernel wins
+// once the queries no longer spread over idle CUs.  18,016 keys in 8 splits, 16 queries:
+// 95 -> 71 us, 8 queries (256 workgroups): 64, not 71; 32 splits, 16 queries: 97 -> 26.
+// Splits of a tile or two: 9.9, not 10.4, with 512 workgroups, 13.7 -> 11.8 with 1,024.
+static int q8_split_mq(int gqa, int num_kv, int sub_n, int k_splits, int m) {
+  const long old_wgs = (long)num_kv * k_splits * sub_n;
+  if (sub_n == 1 || old_wgs <= (m < 192 ? 512 : 256)) return 0;
+  const SplitMq narrow = split_mq(gqa, num_kv, sub_n, k_splits, 32);
+  return narrow.wgs <= 256 ? narrow.queries : split_mq(gqa, num_kv, sub_n, k_splits, 64).queries;
+}
+
 int qkv_attn_split_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block_tq3* v,
                        float* part_m, float* part_l, float* part_o, int num_q, int num_kv,
                        int head_dim, int start_pos, int sub_n, int sub_n_max,
@@ -328,6 +373,12 @@ int qkv_attn_split_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_bloc
   a.part_m = part_m;
   a.part_l = part_l;
   a.part_o = part_o;
+  const int mq_queries = tq3_split_mq(num_q / num_kv, num_kv, sub_n, k_splits, split_keys(active_end_max, k_splits));
+  if (mq_queries) {
+    a.chunk_keys = split_keys(active_end_max, k_splits);
+    a.qpw = mq_queries;
+    return launch_status(qkv::launch_mq_split(a, true, stream));
+  }
   return launch_status(qkv::launch_tq3_attn(a, 1, nullptr, stream));
 }
 
@@ -483,6 +534,12 @@ int qkv_attn_split_q8(const uint16_t* q, const qkv_block_q8* k, const qkv_block_
   a.part_m = part_m;
   a.part_l = part_l;
   a.part_o = part_o;
+  a.chunk_keys = split_keys(active_end_max, k_splits);
+  const int mq_queries = q8_split_mq(num_q / num_kv, num_kv, sub_n, k_splits, a.chunk_keys);
+  if (mq_queries) {
+    a.qpw = mq_queries;
+    return launch_status(qkv::launch_mq_split(a, false, stream));
+  }
   return launch_status(qkv::launch_q8_attn_split(a, stream));
 }
 

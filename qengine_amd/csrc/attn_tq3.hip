@@ -246,74 +246,97 @@ __device__ __forceinline__ void value_steps(const uint8_t* lds, uint32_t (&ac)[4
   }
 }
 
-// Registers of one 64-key tile.  Buffer loads: offsets are 32-bit and reads
+// Registers of one 64-key tile, as loaded: unit i of the lane is piece lane & 3 of
+// block lane >> 5 of the row of key 8 i + ((lane >> 2) & 7) -- the 16 bytes from byte
+// 12 (lane & 3) of the 52-byte block on, i.e. the code groups 4 (lane & 3) .. + 3 in
+// dwords 1..3 and, in piece 0, the block's norm in dword 0.  Four lanes read one
+// block's 52 bytes: the cache looks up a third of the lines it does with a row or a
+// strided piece per lane (1.7 million lookups of a cycle each and CU for 18,016 keys in
+// 8 splits bound that launch: 27 us).  Buffer loads: offsets are 32-bit and reads
 // past the cache extent (num_records) return zero, so partial tiles need no
 // branches; keys in [hi, extent) are read and masked out of the softmax.
 struct TileRegs {
-  u4_t vr[6];            // value row of key ts+lane (dwords 0..23)
-  u2_t vr6;              // dwords 24..25
-  uint32_t kq[4][2][3];  // key code groups 4*row..4*row+3, group g, block j
-  float kn[4][2];        // key block norms, group g, block j
+  u4_t k[8], v[8];
 };
+__device__ __forceinline__ int unit_key8(int lane) { return (lane >> 2) & 7; }
 
 // prow: cache row of the tile's first key (64 consecutive rows, wave-uniform);
 // the buffer resources are rebased at that row (64-bit byte offset)
-__device__ __forceinline__ void load_tile_keys(const AttnArgs& p, int prow, int nkv, int h, int row, int col,
-                                               TileRegs& tr) {
+template <int FROM, int TO>   // units FROM .. TO - 1
+__device__ __forceinline__ void load_tile_part(const uint32_t* base, uint64_t bytes, int prow, int nkv, int h,
+                                               int lane, u4_t (&r)[8]) {
   const uint64_t off0 = (uint64_t)(uint32_t)prow * (uint32_t)nkv * 104u;
-  const __amdgpu_buffer_rsrc_t rk = cache_rsrc(p.k, off0, p.kv_bytes);
-  // keys first (group by group): the score MFMAs of group g only wait for
-  // group g, and values arrive while the scores are computed
+  const __amdgpu_buffer_rsrc_t rs = cache_rsrc(base, off0, bytes);
+  asm volatile("" : "+v"(lane));   // (the offsets are formed per tile, not held in registers)
+  const uint32_t unit = (uint32_t)(unit_key8(lane) * nkv + h) * 104u + 52u * (uint32_t)(lane >> 5) +
+                        12u * (uint32_t)(lane & 3);
 #pragma unroll
-  for (int g = 0; g < 4; g++) {
-    const uint32_t krow = (uint32_t)((16 * g + col) * nkv + h) * 104u;
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const u3_t c = __builtin_amdgcn_raw_buffer_load_b96(rk, krow + 52 * j + 4 + 12 * row, 0, 0);
-      tr.kq[g][j][0] = c[0];
-      tr.kq[g][j][1] = c[1];
-      tr.kq[g][j][2] = c[2];
-      tr.kn[g][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, krow + 52 * j, 0, 0));
-    }
-  }
+  for (int i = FROM; i < TO; i++)
+    r[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, unit + (uint32_t)(i * 8 * nkv) * 104u, 0, 0);
+}
+template <int FROM = 0, int TO = 8>
+__device__ __forceinline__ void load_tile_keys(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRegs& tr) {
+  load_tile_part<FROM, TO>(p.k, p.kv_bytes, prow, nkv, h, lane, tr.k);
 }
 __device__ __forceinline__ void load_tile_values(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRegs& tr) {
-  const uint64_t off0 = (uint64_t)(uint32_t)prow * (uint32_t)nkv * 104u;
-  const __amdgpu_buffer_rsrc_t rv = cache_rsrc(p.v, off0, p.kv_bytes);
-  const uint32_t vrow = (uint32_t)(lane * nkv + h) * 104u;
-#pragma unroll
-  for (int i = 0; i < 6; i++) tr.vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, vrow + 16 * i, 0, 0);
-  tr.vr6 = __builtin_amdgcn_raw_buffer_load_b64(rv, vrow + 96, 0, 0);
+  load_tile_part<0, 8>(p.v, p.kv_bytes, prow, nkv, h, lane, tr.v);
 }
-__device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, int h, int lane, int row, int col,
-                                          TileRegs& tr) {
-  load_tile_keys(p, prow, nkv, h, row, col, tr);
+// keys first: values arrive while the scores are computed
+__device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRegs& tr) {
+  load_tile_keys(p, prow, nkv, h, lane, tr);
   load_tile_values(p, prow, nkv, h, lane, tr);
 }
 
 // The encoded new key (4 x 13 dwords at nr) written over the registers of
-// the tile that holds it, r = its index in the tile: lanes (row, col = r & 15)
-// of its 16-key group take its key code pieces and norms, lane r its value row
-// (constant register indices).
-__device__ __forceinline__ void patch_new_key(TileRegs& tr, const uint32_t* nr, int r, int lane, int row,
-                                              int col) {
-  const int g = r >> 4;
-  if (col == (r & 15)) {
+// the tile that holds it, r = its index in the tile (constant register indices).
+__device__ __forceinline__ void patch_new_key(TileRegs& tr, const uint32_t* nr, int r, int lane) {
+  if (unit_key8(lane) == (r & 7)) {
+    const uint32_t* k = nr + 13 * (lane >> 5) + 3 * (lane & 3);
+    const u4_t nk = {k[0], k[1], k[2], k[3]}, nv = {k[26], k[27], k[28], k[29]};
 #pragma unroll
-    for (int G = 0; G < 4; G++) {
-#pragma unroll
-      for (int j = 0; j < 2; j++) {
-        tr.kq[G][j][0] = g == G ? nr[13 * j + 1 + 3 * row] : tr.kq[G][j][0];
-        tr.kq[G][j][1] = g == G ? nr[13 * j + 2 + 3 * row] : tr.kq[G][j][1];
-        tr.kq[G][j][2] = g == G ? nr[13 * j + 3 + 3 * row] : tr.kq[G][j][2];
-        tr.kn[G][j] = g == G ? __uint_as_float(nr[13 * j]) : tr.kn[G][j];
-      }
+    for (int i = 0; i < 8; i++) {
+      tr.k[i] = i == r >> 3 ? nk : tr.k[i];
+      tr.v[i] = i == r >> 3 ? nv : tr.v[i];
     }
   }
-  if (lane == r) {
+}
+
+// A tile's key units pass through the wave's staging area (before its value codes
+// take it) to the lanes whose score operands they are: key r's piece c of 16 bytes
+// (c = 4 block + piece) at 128 r + 16 (c ^ f(r)), where f(r) = 4 ((r >> 1) & 1) +
+// ((r >> 2) & 3) gives both the 16 lanes of a store (4 keys, 4 pieces) and those of a
+// read (16 keys, one piece) 16 different bank groups.
+__device__ __forceinline__ void stage_keys(uint8_t* st, int lane, const u4_t (&k)[8], float scale2) {
+  const int key8 = unit_key8(lane), c = 4 * (lane >> 5) + (lane & 3);
+  const int at = 128 * key8 + 16 * (c ^ (4 * ((key8 >> 1) & 1) + (key8 >> 2)));
 #pragma unroll
-    for (int i = 0; i < 6; i++) tr.vr[i] = u4_t{nr[26 + 4 * i], nr[27 + 4 * i], nr[28 + 4 * i], nr[29 + 4 * i]};
-    tr.vr6 = u2_t{nr[50], nr[51]};
+  for (int i = 0; i < 8; i++) *reinterpret_cast<u4_t*>(st + (at ^ (32 * (i & 1))) + 1024 * i) = k[i];
+  if ((lane & 3) == 0) {
+    // key norms carry the softmax scale and undo the table scale
+    float* kn = reinterpret_cast<float*>(st) + kStKn + (lane >> 5) * kKeyPitch + key8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) kn[8 * i] = __uint_as_float(k[i][0]) * scale2;
+  }
+}
+// Byte of piece `row` of block 0 of key `col` (block 1: ^ 64; key 16 g + col: + 2048 g).
+__device__ __forceinline__ int staged_key(int row, int col) {
+  return 128 * col + 16 * (row ^ (4 * ((col >> 1) & 1) + (col >> 2)));
+}
+// Value codes, one dword per 8-dim group and key, and norms.
+__device__ __forceinline__ void stage_values(float* st, int lane, const u4_t (&v)[8]) {
+  const int key8 = unit_key8(lane), j = lane >> 5, pc = lane & 3;
+  uint32_t* d = reinterpret_cast<uint32_t*>(st) + kStCodes + (16 * j + 4 * pc) * kKeyPitch + key8;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    d[8 * i] = v[i][1];
+    d[8 * i + kKeyPitch] = __builtin_amdgcn_alignbyte(v[i][2], v[i][1], 3);
+    d[8 * i + 2 * kKeyPitch] = __builtin_amdgcn_alignbyte(v[i][3], v[i][2], 2);
+    d[8 * i + 3 * kKeyPitch] = v[i][3] >> 8;
+  }
+  if (pc == 0) {
+    float* vn = st + kStVn + j * kKeyPitch + key8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) vn[8 * i] = __uint_as_float(v[i][0]);
   }
 }
 
@@ -583,7 +606,7 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   __builtin_amdgcn_s_waitcnt(0);
   QKV_STAMP(kPhQuery);
   TileRegs tr;
-  if (wave < 4) load_tile(p, wave_tile_row(ts0), p.num_kv, h, lane, row, col, tr);
+  if (wave < 4) load_tile(p, wave_tile_row(ts0), p.num_kv, h, lane, tr);
   // centroid-pair table: entry e = (centroid[e & 7], centroid[(e >> 3) & 7])
   // as fp16, from immediates (wave-uniform values); wave w writes every lane's
   // copy of entries 32w .. 32w+31
@@ -706,7 +729,7 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   // before the second (waves 4..7), so that across the chip the first waves'
   // tiles arrive in the first half of the stream and are computed while the
   // second waves' tiles are still in flight.
-  if (wave >= 4) load_tile(p, wave_tile_row(ts0), p.num_kv, h, lane, row, col, tr);
+  if (wave >= 4) load_tile(p, wave_tile_row(ts0), p.num_kv, h, lane, tr);
   // qa[s], slice s = 4j+u: column `col`, element i = dim 128j + 8(4*row+u) + i
   h8_t qa[8];
   {
@@ -735,71 +758,58 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   f4_t acc[16];
 
   float* st = reinterpret_cast<float*>(lds + kLdsStage + wave * kStageBytes);
-  uint32_t* stu = reinterpret_cast<uint32_t*>(st);
+  const uint32_t* stu = reinterpret_cast<const uint32_t*>(st);
 
-  // The split forms, whose workgroups are few and walk several tiles, load the next
-  // tile's keys ahead (18,016 keys in 8 splits, GQA 6: 33.0 -> 29.4 us with the merge).
-  // The fast path has one tile per wave at most contexts and two waves per SIMD to
-  // overlap at the others: nothing at 131,072 keys, and paged slots lose (102 -> 109 us).
-  constexpr bool kPrefetch = MODE >= 1;
+  // Key units of the next tile that are loaded ahead, during the softmax and the
+  // values: all (131,072 keys: 31.6 -> 31.0 us, 65,000: 20.6 -> 20.1), or the half
+  // that the chained form has registers for (all: 35 spills, 35.7 -> 41.7 us).
+  constexpr int kAhead = CHAIN ? 4 : 8;
   int next_row = 0;   // cache row of the wave's next tile, whose keys are on their way
   // One 64-key tile.  The wave's first tile is a separate instance: its loads
   // were issued with the setup, and its accumulators start at zero.
   // next: first key of the wave's next tile, < 0 if this is its last.
   auto tile_body = [&](auto first_tag, int ts, int next) {
     constexpr bool first = decltype(first_tag)::value;
-    auto& kq = tr.kq;
-    auto& kn = tr.kn;
+    // (opaque lane index: the staging addresses are formed here, not held in
+    // registers through the tile)
+    int lane_o = lane;
+    asm volatile("" : "+v"(lane_o));
+    stage_keys(reinterpret_cast<uint8_t*>(st), lane_o, tr.k, scale2);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
     // ---------------- scores: D rows = keys 16g + 4*row + r, D col = head `col` ----------------
     f4_t sa[4][2];
+    {
+      const uint8_t* ks = reinterpret_cast<const uint8_t*>(st) + staged_key(lane_o >> 4, lane_o & 15);
+      const uint8_t* ks1 = reinterpret_cast<const uint8_t*>(st) + (staged_key(lane_o >> 4, lane_o & 15) ^ 64);
+      u4_t n0 = *reinterpret_cast<const u4_t*>(ks), n1 = *reinterpret_cast<const u4_t*>(ks1);
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-      sa[g][0] = f4_t{0.f, 0.f, 0.f, 0.f};
-      sa[g][1] = f4_t{0.f, 0.f, 0.f, 0.f};
-      score_group<0, CHAIN>(lds, ac, kq[g][0], kq[g][1], qa, qlo, group_operand<0>(lds, ac, kq[g][0]),
-                            group_operand<0>(lds, ac, kq[g][1]), sa[g][0], sa[g][1]);
+      for (int g = 0; g < 4; g++) {
+        const uint32_t k0[3] = {n0[1], n0[2], n0[3]}, k1[3] = {n1[1], n1[2], n1[3]};
+        if (g < 3) {   // the next group's codes ahead of this group's products
+          n0 = *reinterpret_cast<const u4_t*>(ks + 2048 * (g + 1));
+          n1 = *reinterpret_cast<const u4_t*>(ks1 + 2048 * (g + 1));
+        }
+        sa[g][0] = f4_t{0.f, 0.f, 0.f, 0.f};
+        sa[g][1] = f4_t{0.f, 0.f, 0.f, 0.f};
+        score_group<0, CHAIN>(lds, ac, k0, k1, qa, qlo, group_operand<0>(lds, ac, k0), group_operand<0>(lds, ac, k1),
+                              sa[g][0], sa[g][1]);
+      }
     }
 
     if constexpr (first) QKV_STAMP(kPhScores);
-    // ---------------- staging: key norms, value rows (lane = key ts + lane) ----------------
-    if (row == 0) {
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        // key norms carry the softmax scale and undo the table scale
-        st[kStKn + 16 * g + col] = kn[g][0] * scale2;
-        st[kStKn + kKeyPitch + 16 * g + col] = kn[g][1] * scale2;
-      }
-    }
-    {
-      uint32_t d[27];
-#pragma unroll
-      for (int i = 0; i < 6; i++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) d[4 * i + e] = tr.vr[i][e];
-      d[24] = tr.vr6[0];
-      d[25] = tr.vr6[1];
-      d[26] = 0u;
-#pragma unroll
-      for (int j = 0; j < 2; j++) {
-        stu[kStVn + j * kKeyPitch + lane] = d[13 * j];
-#pragma unroll
-        for (int g = 0; g < 16; g++) {
-          // code group g of block j: bytes 3g..3g+2 of the codes (dword 13j+1 on)
-          const int w = 13 * j + 1 + ((3 * g) >> 2), sh = (3 * g) & 3;
-          stu[kStCodes + (16 * j + g) * kKeyPitch + lane] =
-              sh ? __builtin_amdgcn_alignbyte(d[w + 1], d[w], sh) : d[w];
-        }
-      }
-    }
+    // ---------------- staging: value codes and norms ----------------
+    stage_values(st, lane_o, tr.v);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     // the key registers are free: the next tile's keys fly during the softmax and the
     // value products (its values, during its scores: there are no registers for both)
-    if (kPrefetch && next >= 0) {
+    if (next >= 0) {
       next_row = wave_tile_row(next);
-      load_tile_keys(p, next_row, p.num_kv, h, row, col, tr);
+      load_tile_keys<0, kAhead>(p, next_row, p.num_kv, h, lane, tr);
     }
 
     // dense is wave-uniform: the common full tile (every key visible to every
@@ -899,15 +909,13 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   } else if (ts0 < hi) {
     auto following = [&](int ts) { return ts + kStep < hi ? ts + kStep : -1; };
     if (APPEND && fa_wave == wave && ts0 <= p.start_pos && p.start_pos < ts0 + kTile)
-      patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts0, lane, row, col);
+      patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts0, lane);
     tile_body(std::true_type{}, ts0, following(ts0));
     for (int ts = ts0 + kStep; ts < hi; ts += kStep) {
-      if constexpr (kPrefetch)
-        load_tile_values(p, next_row, p.num_kv, h, lane, tr);
-      else
-        load_tile(p, wave_tile_row(ts), p.num_kv, h, lane, row, col, tr);
+      load_tile_keys<kAhead, 8>(p, next_row, p.num_kv, h, lane, tr);
+      load_tile_values(p, next_row, p.num_kv, h, lane, tr);
       if (APPEND && fa_wave == wave && ts <= p.start_pos && p.start_pos < ts + kTile)
-        patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts, lane, row, col);
+        patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts, lane);
       tile_body(std::false_type{}, ts, following(ts));
     }
   } else {

@@ -287,6 +287,78 @@ __device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, 
   load_tile_values(p, prow, nkv, h, lane, tr);
 }
 
+// The same tile with a lane's own operands: strided 12-byte key pieces and whole value
+// rows, which need no pass through the LDS before the scores.  For the split forms
+// (MODE >= 1): their few workgroups walk many tiles in a row, where that pass is part
+// of every round and the cache lookups are not the bound (one query in 8 splits,
+// 64,533 keys: 81.6 us, 89.7 in units; 18,016: 29.4, 30.7).
+struct TileRows {
+  u4_t vr[6];            // value row of key ts+lane (dwords 0..23)
+  u2_t vr6;              // dwords 24..25
+  uint32_t kq[4][2][3];  // key code groups 4*row..4*row+3, group g, block j
+  float kn[4][2];        // key block norms, group g, block j
+};
+template <int FROM = 0, int TO = 8>
+__device__ __forceinline__ void load_tile_keys(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRows& tr) {
+  if constexpr (FROM < TO) {
+    const int row = lane >> 4, col = lane & 15;
+    const __amdgpu_buffer_rsrc_t rk = cache_rsrc(p.k, (uint64_t)(uint32_t)prow * (uint32_t)nkv * 104u, p.kv_bytes);
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const uint32_t krow = (uint32_t)((16 * g + col) * nkv + h) * 104u;
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        const u3_t c = __builtin_amdgcn_raw_buffer_load_b96(rk, krow + 52 * j + 4 + 12 * row, 0, 0);
+        tr.kq[g][j][0] = c[0];
+        tr.kq[g][j][1] = c[1];
+        tr.kq[g][j][2] = c[2];
+        tr.kn[g][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, krow + 52 * j, 0, 0));
+      }
+    }
+  }
+}
+__device__ __forceinline__ void load_tile_values(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRows& tr) {
+  const __amdgpu_buffer_rsrc_t rv = cache_rsrc(p.v, (uint64_t)(uint32_t)prow * (uint32_t)nkv * 104u, p.kv_bytes);
+  const uint32_t vrow = (uint32_t)(lane * nkv + h) * 104u;
+#pragma unroll
+  for (int i = 0; i < 6; i++) tr.vr[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, vrow + 16 * i, 0, 0);
+  tr.vr6 = __builtin_amdgcn_raw_buffer_load_b64(rv, vrow + 96, 0, 0);
+}
+__device__ __forceinline__ void load_tile(const AttnArgs& p, int prow, int nkv, int h, int lane, TileRows& tr) {
+  load_tile_keys(p, prow, nkv, h, lane, tr);
+  load_tile_values(p, prow, nkv, h, lane, tr);
+}
+// Staging of a tile in rows: key norms, value codes and norms.
+__device__ __forceinline__ void stage_rows(float* st, int lane, const TileRows& tr, float scale2) {
+  const int row = lane >> 4, col = lane & 15;
+  uint32_t* stu = reinterpret_cast<uint32_t*>(st);
+  if (row == 0) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      st[kStKn + 16 * g + col] = tr.kn[g][0] * scale2;
+      st[kStKn + kKeyPitch + 16 * g + col] = tr.kn[g][1] * scale2;
+    }
+  }
+  uint32_t d[27];
+#pragma unroll
+  for (int i = 0; i < 6; i++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) d[4 * i + e] = tr.vr[i][e];
+  d[24] = tr.vr6[0];
+  d[25] = tr.vr6[1];
+  d[26] = 0u;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    stu[kStVn + j * kKeyPitch + lane] = d[13 * j];
+#pragma unroll
+    for (int g = 0; g < 16; g++) {
+      // code group g of block j: bytes 3g..3g+2 of the codes (dword 13j+1 on)
+      const int w = 13 * j + 1 + ((3 * g) >> 2), sh = (3 * g) & 3;
+      stu[kStCodes + (16 * j + g) * kKeyPitch + lane] = sh ? __builtin_amdgcn_alignbyte(d[w + 1], d[w], sh) : d[w];
+    }
+  }
+}
+
 // The encoded new key (4 x 13 dwords at nr) written over the registers of
 // the tile that holds it, r = its index in the tile (constant register indices).
 __device__ __forceinline__ void patch_new_key(TileRegs& tr, const uint32_t* nr, int r, int lane) {
@@ -605,7 +677,8 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   // and the rotation; waves 4..7 issue theirs after the setup barrier.
   __builtin_amdgcn_s_waitcnt(0);
   QKV_STAMP(kPhQuery);
-  TileRegs tr;
+  constexpr bool kUnits = MODE == 0;   // tiles in units, or in rows (TileRows)
+  std::conditional_t<kUnits, TileRegs, TileRows> tr;
   if (wave < 4) load_tile(p, wave_tile_row(ts0), p.num_kv, h, lane, tr);
   // centroid-pair table: entry e = (centroid[e & 7], centroid[(e >> 3) & 7])
   // as fp16, from immediates (wave-uniform values); wave w writes every lane's
@@ -774,14 +847,16 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
     // registers through the tile)
     int lane_o = lane;
     asm volatile("" : "+v"(lane_o));
-    stage_keys(reinterpret_cast<uint8_t*>(st), lane_o, tr.k, scale2);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if constexpr (kUnits) {
+      stage_keys(reinterpret_cast<uint8_t*>(st), lane_o, tr.k, scale2);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
 
     // ---------------- scores: D rows = keys 16g + 4*row + r, D col = head `col` ----------------
     f4_t sa[4][2];
-    {
+    if constexpr (kUnits) {
       const uint8_t* ks = reinterpret_cast<const uint8_t*>(st) + staged_key(lane_o >> 4, lane_o & 15);
       const uint8_t* ks1 = reinterpret_cast<const uint8_t*>(st) + (staged_key(lane_o >> 4, lane_o & 15) ^ 64);
       u4_t n0 = *reinterpret_cast<const u4_t*>(ks), n1 = *reinterpret_cast<const u4_t*>(ks1);
@@ -797,11 +872,22 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
         score_group<0, CHAIN>(lds, ac, k0, k1, qa, qlo, group_operand<0>(lds, ac, k0), group_operand<0>(lds, ac, k1),
                               sa[g][0], sa[g][1]);
       }
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        sa[g][0] = f4_t{0.f, 0.f, 0.f, 0.f};
+        sa[g][1] = f4_t{0.f, 0.f, 0.f, 0.f};
+        score_group<0, CHAIN>(lds, ac, tr.kq[g][0], tr.kq[g][1], qa, qlo, group_operand<0>(lds, ac, tr.kq[g][0]),
+                              group_operand<0>(lds, ac, tr.kq[g][1]), sa[g][0], sa[g][1]);
+      }
     }
 
     if constexpr (first) QKV_STAMP(kPhScores);
     // ---------------- staging: value codes and norms ----------------
-    stage_values(st, lane_o, tr.v);
+    if constexpr (kUnits)
+      stage_values(st, lane_o, tr.v);
+    else
+      stage_rows(st, lane_o, tr, scale2);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -908,14 +994,16 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
     }
   } else if (ts0 < hi) {
     auto following = [&](int ts) { return ts + kStep < hi ? ts + kStep : -1; };
-    if (APPEND && fa_wave == wave && ts0 <= p.start_pos && p.start_pos < ts0 + kTile)
-      patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts0, lane);
+    if constexpr (APPEND)
+      if (fa_wave == wave && ts0 <= p.start_pos && p.start_pos < ts0 + kTile)
+        patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts0, lane);
     tile_body(std::true_type{}, ts0, following(ts0));
     for (int ts = ts0 + kStep; ts < hi; ts += kStep) {
       load_tile_keys<kAhead, 8>(p, next_row, p.num_kv, h, lane, tr);
       load_tile_values(p, next_row, p.num_kv, h, lane, tr);
-      if (APPEND && fa_wave == wave && ts <= p.start_pos && p.start_pos < ts + kTile)
-        patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts, lane);
+      if constexpr (APPEND)
+        if (fa_wave == wave && ts <= p.start_pos && p.start_pos < ts + kTile)
+          patch_new_key(tr, reinterpret_cast<const uint32_t*>(lds + kLdsNewRow), p.start_pos - ts, lane);
       tile_body(std::false_type{}, ts, following(ts));
     }
   } else {

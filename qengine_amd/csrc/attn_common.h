@@ -365,6 +365,8 @@ hipError_t launch_q8k_tq3v_attn_fast(const AttnArgs& a, uint16_t* out, hipStream
 hipError_t launch_q8_attn_fast_append(const AttnArgs& a, uint16_t* out, hipStream_t stream);
 // multi-query decode (attn_mq.hip): TQ3 or Q8_0 keys, TQ3 or Q8_0 values (TQ3 with TQ3 keys)
 hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* out, hipStream_t stream);
+// The merge of a launch's records as a launch of its own (attn_merge.hip); rotate: TQ3 values.
+hipError_t launch_record_merge(const AttnArgs& a, bool rotate, uint16_t* out, hipStream_t stream);
 hipError_t launch_mq_split(const AttnArgs& a, bool tq3, hipStream_t stream);
 hipError_t launch_split_merge(const float* m, const float* l, const float* o, uint16_t* out,
                               int num_q, int sub_n, int sub_n_max, int k_splits,

@@ -4,9 +4,12 @@
 // splits; splits with non-finite m or l <= 0 are skipped; out = sum w*o /
 // sum w*l with w = exp(m_s - M), 0 when the sum is 0; fp16 output
 // [t][q_head][256].  One workgroup per (q head, t), one thread per dim.
+//
+// record_merge_kernel is the same merge over the records of a decode launch.
 #include <algorithm>
 
 #include "attn_common.h"
+#include "attn_fastmerge.h"
 #include "qkv_launch.h"
 #include "qkv_device.h"
 
@@ -94,6 +97,77 @@ hipError_t launch_ws_status(const void* workspace, int* status, int ok_value, in
                             hipStream_t stream) {
   hipLaunchKernelGGL(ws_status_kernel, dim3(1), dim3(64), 0, stream, static_cast<const int*>(workspace),
                      status, ok_value, timeout_value);
+  return hipGetLastError();
+}
+
+// The records of a multi-query decode launch (attn_mq.hip), which precedes this one on
+// the stream, to the output: one workgroup per (query, q head, 128-dim block) unit.  A
+// launch of its own, because every workgroup of that one writes records that units all
+// over the grid need: workgroups that wait for records in the launch that writes them
+// hold the CUs that its other workgroups, or those of a launch on another stream, are
+// still to run on.  The records are complete
+// here, so their scalars and rows are loaded at once, one memory round trip; the
+// arguments are scalars that arrive in registers with the wave (attn_common.h) and the
+// unit comes from the three grid dimensions, without a division.
+// A tag that is missing all the same (the workspace is in use by another call, or the
+// poll limit is 0) is the timeout of the in-launch merges: NaN rows and the sticky error.
+// Against the merge within attn_mq.hip's launch, us for the call, TQ3, 16 q heads:
+// 8 queries over 301 keys 15.0 -> 13.0, 5 over 18,016 21.2 -> 20.0, 16 over 32,767
+// 36.4 -> 36.4; Q8_0, 16 over 4,096 19.1 -> 18.4, 2 over 18,016 20.9 -> 21.8.
+constexpr int kRecThreads = 256;
+template <bool ROTATE>
+__global__ __launch_bounds__(kRecThreads) void record_merge_kernel(float* ws_ml, float* ws_o, int* ws_header,
+                                                                   uint16_t* out, uint32_t ws_ml_bytes,
+                                                                   uint32_t ws_o_bytes, int num_q, int sub_n,
+                                                                   int n, int spin_limit) {
+  using ML = MergeLayout<kRecThreads>;
+  __shared__ __attribute__((aligned(16))) float red[ML::kRedFloats];
+  __shared__ f2_t mls[128];
+  __shared__ int vote[ML::kWaves];
+  AttnArgs p{};
+  p.num_q = num_q;
+  p.sub_n = sub_n;
+  p.n_slots = n;
+  const int tid = threadIdx.x;
+  const int t = blockIdx.x, qh = blockIdx.y, blk = blockIdx.z;
+  const long base = rec_index(p, qh, t, 0);
+  const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(ws_ml, 0, ws_ml_bytes, kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(ws_o, 0, ws_o_bytes, kBufferRsrcWord3);
+  const bool poisoned = __hip_atomic_load(ws_header + kWsErrorWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  f4_t r = {0.f, 0.f, 0.f, 0.f};
+  if (tid < n)
+    r = __builtin_amdgcn_raw_buffer_load_b128(rml, (uint32_t)((base + tid) * kRecMlBytes), 0, kCoherent);
+  f4_t v[ML::kRecPerThread];
+#pragma unroll
+  for (int i = 0; i < ML::kRecPerThread; i++) {
+    const int c = (tid >> 5) + ML::kSlices * i;
+    v[i] = c < n ? __builtin_amdgcn_raw_buffer_load_b128(
+                       ro, (uint32_t)(((base + c) * 256 + blk * 128 + 4 * (tid & 31)) * 4), 0, kCoherent)
+                 : f4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  if (poisoned) {   // (uniform) left inconsistent by an earlier timeout: NaN rows until it is reset
+    write_nan_unit(p, t, qh, blk, out);
+    return;
+  }
+  const bool seen = tid < n && spin_limit > 0 && __float_as_uint(blk ? r[3] : r[2]) == kTagValid;
+  if (tid < n) mls[tid] = f2_t{r[0], r[1]};
+  if (seen)   // clear: the state that the next launch on this workspace starts from
+    __builtin_amdgcn_raw_buffer_store_b32(0u, rml, (uint32_t)((base + tid) * kRecMlBytes + 8 + 4 * blk), 0,
+                                          kCoherent);
+  if (!block_and<kRecThreads>(seen || tid >= n, vote)) {
+    write_nan_unit(p, t, qh, blk, out);
+    if (tid == 0)
+      __hip_atomic_store(ws_header + kWsErrorWord, kWsErrorTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  fold_unit<kRecThreads, ROTATE>(red, mls, p, v, n, qh, t, blk, out);
+}
+
+hipError_t launch_record_merge(const AttnArgs& a, bool rotate, uint16_t* out, hipStream_t stream) {
+  const dim3 grid(a.sub_n, a.num_q, 2), block(kRecThreads);
+  auto* kernel = rotate ? record_merge_kernel<true> : record_merge_kernel<false>;
+  hipLaunchKernelGGL(kernel, grid, block, 0, stream, a.ws_ml, a.ws_o, a.ws_header, out, a.ws_ml_bytes, a.ws_o_bytes,
+                     a.num_q, a.sub_n, a.n_chunks, a.spin_limit);
   return hipGetLastError();
 }
 

@@ -1,4 +1,4 @@
-// attn_mq.hip -- single-launch decode of multi-query calls (verify blocks):
+// attn_mq.hip -- decode of multi-query calls (verify blocks):
 // every cache tile is read once for up to 64 (query, head) columns (gfx950).
 //
 // Reference semantics: the split kernels with sub_n > 1 and their merge
@@ -29,9 +29,8 @@
 //            dims of the records itself.
 // One barrier per tile: the scores of tile t + 1 follow the value product of
 // tile t in the same interval (three staging buffers, two of probabilities).
-// Records are merged across workgroups as in the
-// other fast paths (attn_fastmerge.h).
-#include <algorithm>
+// The records are merged by a launch of their own (attn_merge.hip): no workgroup
+// waits for another, so a call completes on whatever part of the GPU is free.
 #include <type_traits>
 
 #include "attn_common.h"
@@ -69,7 +68,6 @@ constexpr float kSlack = VT ? 8.0f : 14.0f;
 template <bool VT>
 constexpr float kHead = VT ? 0.0f : 6.0f;
 constexpr float kNoRef = -1e30f;
-constexpr int kMaxWgs = 256;   // one workgroup per CU
 
 // Centroid-pair table: entry e (two 3-bit codes) of lane L at byte e * 256 + 4 * L
 // (64 entries, so indexes are clean 6-bit values).
@@ -96,9 +94,7 @@ struct MqLds {
   // setup (TQ3 keys): rotated queries, fp16 rounding and remainder [64 columns][512 B] each
   static constexpr int kQhi = kK, kQlo = kK + 64 * 512;
   // after the tile loop
-  static constexpr int kRed = 0;                          // mergers
-  static constexpr int kMls = kRed + kWaves * 128 * 4;
-  static constexpr int kSum = kMls + 256 * 8;             // [4][64] sums, [64] maxima, [64] record indices
+  static constexpr int kSum = 0;                          // [4][64] sums, [64] maxima, [64] record indices
   static constexpr int kRowPitch = kHD + 4;               // SPLIT: rows to rotate back, kSum's maxima in between
   static constexpr int kRows = kSum + 10 * 64 * 4;
   static_assert(kRows + 32 * kRowPitch * 4 <= kEnd, "rows to rotate back (NG = 2)");
@@ -278,7 +274,7 @@ __device__ __forceinline__ uint32_t pair_read(const uint8_t* lds, uint32_t w, ui
 // in natural-log units, sum, unnormalised row in the caller's coordinates) go to
 // part_m / part_l / part_o.
 template <bool KT, bool VT, int NG, bool SPLIT>
-__global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARAMS, AttnArgs pin, uint16_t* out) {
+__global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARAMS, AttnArgs pin) {
   QKV_ATTN_LEAD_APPLY(p, pin);
   static_assert(!KT || VT, "TQ3 keys come with TQ3 values");
   using L = MqLds<KT, VT>;
@@ -289,17 +285,15 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   const int gqa = __builtin_amdgcn_readfirstlane(p.num_q / p.num_kv);
   // work id, XCD-aware: the num_kv workgroups of one (query block, chunk) share an XCD
   int h, t0, chunk;
-  bool has_work;
   {
     const int Lid = blockIdx.x;
     const int xcd = Lid & 7, r = Lid >> 3;
     h = r % p.num_kv;
     const int g = (r / p.num_kv) * 8 + xcd;
     const int groups = (p.sub_n + p.qpw - 1) / p.qpw;
-    has_work = g < groups * p.n_chunks;
-    if (SPLIT && !has_work) return;
-    const int tq = has_work ? g / p.n_chunks : 0;
-    chunk = has_work ? g - tq * p.n_chunks : 0;
+    if (g >= groups * p.n_chunks) return;
+    const int tq = g / p.n_chunks;
+    chunk = g - tq * p.n_chunks;
     t0 = tq * p.qpw;
   }
   const int nq = min(p.qpw, p.sub_n - t0);
@@ -341,13 +335,9 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   __builtin_amdgcn_sched_barrier(0);
   // ---- key range of the workgroup
   const int active_last = p.start_pos + t0 + nq;
-  int lo = 0, hi = 0, hi_first = 0, c_end = 0;
-  if (has_work) {
-    lo = chunk * p.chunk_keys;
-    c_end = !SPLIT && chunk == p.n_chunks - 1 ? active_last : lo + p.chunk_keys;
-    hi = min(c_end, active_last);
-    hi_first = min(c_end, p.start_pos + t0 + 1);
-  }
+  int lo = chunk * p.chunk_keys;
+  const int c_end = !SPLIT && chunk == p.n_chunks - 1 ? active_last : lo + p.chunk_keys;
+  int hi = min(c_end, active_last), hi_first = min(c_end, p.start_pos + t0 + 1);
   lo = __builtin_amdgcn_readfirstlane(lo);
   hi = __builtin_amdgcn_readfirstlane(hi);
   hi_first = __builtin_amdgcn_readfirstlane(hi_first);
@@ -359,7 +349,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   // last query group's workgroups also store them to the caches.
   int new_lo = 0, n_new = 0;
   if constexpr (KT) {
-    if (p.k_new != nullptr && has_work && hi > max(lo, p.start_pos)) {
+    if (p.k_new != nullptr && hi > max(lo, p.start_pos)) {
       new_lo = max(lo, p.start_pos);
       n_new = hi - new_lo;   // <= sub_n <= 64 (the host takes this path only then)
     }
@@ -907,53 +897,45 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   }
   if (tid_e < 64) recs[tid_e] = (int)rec_index(p, h * gqa_m + tid_e % gqa_m, t0 + min(tid_e, cols - 1) / gqa_m, chunk);
   __syncthreads();
-  if (has_work) {
 #pragma unroll
-    for (int g = 0; g < NG; g++) {
+  for (int g = 0; g < NG; g++) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int R = 16 * g + 4 * kb_e + r;
-        if (R < cols)
-          __builtin_amdgcn_raw_buffer_store_b64(f2_t{acc[g][0][r], acc[g][1][r]}, ro,
-                                                (uint32_t)((recs[R] * kHD + 32 * wave + 2 * n_e) * 4), 0, kCoherent);
-      }
+    for (int r = 0; r < 4; r++) {
+      const int R = 16 * g + 4 * kb_e + r;
+      if (R < cols)
+        __builtin_amdgcn_raw_buffer_store_b64(f2_t{acc[g][0][r], acc[g][1][r]}, ro,
+                                              (uint32_t)((recs[R] * kHD + 32 * wave + 2 * n_e) * 4), 0, kCoherent);
     }
-    if (tid_e < cols)
-      __builtin_amdgcn_raw_buffer_store_b64(
-          f2_t{sums[4 * 64 + tid_e], (sums[tid_e] + sums[64 + tid_e]) + (sums[128 + tid_e] + sums[192 + tid_e])}, rml,
-          (uint32_t)(recs[tid_e] * kRecMlBytes), 0, kCoherent);
-    publish_records(p, rml, h, gqa_m, t0, cols, chunk);
-  } else {
-    __syncthreads();   // (the barrier publish_records passes)
   }
-  merge_phase_paired<kThreads, VT>(reinterpret_cast<float*>(lds + L::kRed), reinterpret_cast<f2_t*>(lds + L::kMls), p,
-                                   rml, ro, out);
+  if (tid_e < cols) {
+    const float l = (sums[tid_e] + sums[64 + tid_e]) + (sums[128 + tid_e] + sums[192 + tid_e]);
+    __builtin_amdgcn_raw_buffer_store_b128(
+        u4_t{__float_as_uint(sums[4 * 64 + tid_e]), __float_as_uint(l), kTagValid, kTagValid}, rml,
+        (uint32_t)(recs[tid_e] * kRecMlBytes), 0, kCoherent);
+  }
 }
 
 }  // namespace
 
 template <bool KT, bool VT>
-static void launch_mq(const AttnArgs& a, int n_wg, uint16_t* out, hipStream_t stream) {
+static void launch_mq(const AttnArgs& a, int n_wg, hipStream_t stream) {
   if (a.qpw * (a.num_q / a.num_kv) > 32)
-    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 4, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 4, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
   else
-    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 2, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 2, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
 }
 
 hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* out, hipStream_t stream) {
   const int groups = (a.sub_n + a.qpw - 1) / a.qpw * a.n_chunks;
-  // One round of the GPU holds a merger for every pair of merge units: a short
-  // context, whose chunks are few, gets workgroups that only merge.
-  const int mergers = std::min(a.num_q * a.sub_n, kMaxWgs);
-  const int per = 8 * a.num_kv;
-  const int n_wg = std::max((groups + 7) / 8, (mergers + per - 1) / per) * per;
+  const int n_wg = (groups + 7) / 8 * 8 * a.num_kv;
   if (k_tq3)
-    launch_mq<true, true>(a, n_wg, out, stream);
+    launch_mq<true, true>(a, n_wg, stream);
   else if (v_tq3)
-    launch_mq<false, true>(a, n_wg, out, stream);
+    launch_mq<false, true>(a, n_wg, stream);
   else
-    launch_mq<false, false>(a, n_wg, out, stream);
-  return hipGetLastError();
+    launch_mq<false, false>(a, n_wg, stream);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? e : launch_record_merge(a, v_tq3, out, stream);
 }
 
 // The split API's partials (TQ3 caches: at most 32 columns per workgroup).
@@ -963,11 +945,11 @@ hipError_t launch_mq_split(const AttnArgs& a, bool tq3, hipStream_t stream) {
   const bool wide = a.qpw * (a.num_q / a.num_kv) > 32;
   if (tq3 && wide) return hipErrorInvalidValue;
   if (tq3)
-    hipLaunchKernelGGL((mq_attn_kernel<true, true, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, nullptr);
+    hipLaunchKernelGGL((mq_attn_kernel<true, true, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
   else if (wide)
-    hipLaunchKernelGGL((mq_attn_kernel<false, false, 4, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, nullptr);
+    hipLaunchKernelGGL((mq_attn_kernel<false, false, 4, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
   else
-    hipLaunchKernelGGL((mq_attn_kernel<false, false, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, nullptr);
+    hipLaunchKernelGGL((mq_attn_kernel<false, false, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
   return hipGetLastError();
 }
 

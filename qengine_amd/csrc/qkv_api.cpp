@@ -659,8 +659,8 @@ size_t fast_ws_upto(int num_q, int num_kv, int sub_n, int n_keys, int base, int 
 
 // mq_attn_kernel (attn_mq.hip): queries per workgroup (returned) and chunks.
 // Chunks are whole 64-key tiles, at least two (a chunk pays for its records),
-// at most max_chunks of them; the launch is one round of the GPU.  A call that
-// leaves CUs idle is split over query groups: fewer columns make a tile cheaper
+// at most max_chunks of them; the launch is one round of the GPU, or one chunk
+// per (query group, kv head) where these alone are more.  A call that leaves CUs idle is split over query groups: fewer columns make a tile cheaper
 // and leave each workgroup fewer record rows to write.
 // Costs as measured (131,072 against 65,000 keys): 1.7 us per tile up to 32
 // columns, 2.05 with 64; 64 KB of records per workgroup ~3.2 us.
@@ -847,15 +847,14 @@ size_t qkv_decode_attn_q8_workspace_bytes(int num_q, int num_kv, int sub_n, int 
 // Multi-query calls over Q8_0 keys take the kernel that reads every tile once
 // for up to 64 (query, head) columns (mq_attn_kernel), unless one workgroup
 // per (kv head, query, chunk) fits the GPU in one round: then q8_attn_kernel's
-// shorter chain wins (1,000 keys, 2 to 8 queries: 9.6-9.8 us against
-// 11.6-11.8; 12 queries, 384 workgroups: 12.4 against 12.1; 4,096 keys, 2
-// queries, 272 workgroups: 13.4 against 12.6).  Two of its workgroups share a
-// CU, and with more than 4 heads per column block of the other kernel that
-// second round still wins while the chunks are few (GQA 6 over 1,000 keys, 16
-// queries: 14.2 against 15.3; over 4,096, 2 queries: 13.7 against 12.7).
-bool q8_takes_mq(const FastGeom& g, int num_q, int num_kv, int sub_n) {
-  const long round = num_q / num_kv > 4 && g.n_chunks <= 16 ? 2 * kMaxFastWgs : kMaxFastWgs;
-  return sub_n > 1 && (long)sub_n * g.n_chunks * num_kv > round;
+// shorter chain and its merge in the same launch win (GQA 4, 1,000 keys, 2 and
+// 8 queries: 11.2 and 11.7 us against 12.2 and 12.7; 10 queries, 320
+// workgroups: 14.4 against 13.0; 4,096 keys, 2 queries, 272 workgroups: 14.2
+// against 12.7; GQA 6, 1,000 keys, 16 queries: 16.2 against 14.2).  With TQ3
+// values the two are level there (1,000 keys, 10 queries: 16.6 and 16.8; 5
+// over 2,000: 16.3 and 16.0).
+bool q8_takes_mq(const FastGeom& g, int num_kv, int sub_n) {
+  return sub_n > 1 && (long)sub_n * g.n_chunks * num_kv > kMaxFastWgs;
 }
 
 // Fast path over Q8_0 keys; values Q8_0 (v_tq3 false) or TQ3 (v_tq3 true).
@@ -872,7 +871,7 @@ static int decode_q8_keys(const uint16_t* q, const void* k, const void* v, uint1
   const int n_keys = start_pos + sub_n;
   FastGeom g = fast_geom(num_q, num_kv, sub_n, n_keys, kChunkKeysQ8);
   if (!workspace || workspace_bytes < g.total) return QKV_ERR_WORKSPACE;
-  const bool mq = q8_takes_mq(g, num_q, num_kv, sub_n);
+  const bool mq = q8_takes_mq(g, num_kv, sub_n);
   const int qpw = mq ? mq_geom(g, num_q, num_kv, sub_n, n_keys, g.n_chunks) : 1;
   g.n_slots = g.n_chunks;
   if (!aligned(workspace, 256)) return QKV_ERR_ALIGN;

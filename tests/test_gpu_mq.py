@@ -91,3 +91,81 @@ def test_non_finite_rows_stay_with_the_queries_that_see_them(dev, fmt, plane):
         bad = ~np.isfinite(many)
         assert bad[seen:].any() and np.array_equal(bad, ~np.isfinite(one))
         assert rel_err(np.where(bad, 0.0, one), np.where(bad, 0.0, many)) < TOL
+
+
+def _call(fmt):
+    from qengine_amd import kvcache
+    return {"q8": (kvcache.decode_attn_q8_workspace, kvcache.decode_attn_q8),
+            "mixed": (kvcache.decode_attn_q8k_tq3v_workspace, kvcache.decode_attn_q8k_tq3v),
+            "tq3": (kvcache.decode_attn_tq3_workspace, kvcache.decode_attn_tq3)}[fmt]
+
+
+def _caches(rng, dev, fmt, n, num_kv):
+    k16, v16 = kv_f16(rng, n, num_kv, 256), kv_f16(rng, n, num_kv, 256)
+    return (_dev((O.tq3_encode(k16) if fmt == "tq3" else O.q8_encode(k16)).view(np.uint8), dev),
+            _dev((O.q8_encode(v16) if fmt == "q8" else O.tq3_encode(v16)).view(np.uint8), dev))
+
+
+@pytest.mark.parametrize("fmt", ["q8", "mixed", "tq3"])
+@pytest.mark.parametrize("n,num_q,num_kv,sub_n", [
+    (2048, 16, 4, 1040),    # 260 working workgroups: the first count past 256
+    (2048, 16, 4, 2048),    # no history, two rounds
+    (4000, 64, 8, 300),     # GQA 8
+    (1500, 24, 3, 345),     # 3 kv heads: the grid's rounding to 8 chunks leaves work past id 255
+])
+def test_calls_past_one_round_of_the_gpu(dev, fmt, n, num_q, num_kv, sub_n):
+    """More (query group, kv head) pairs than CUs: the call is several rounds of
+    workgroups, none of which may wait for one that has no CU yet.  Against the
+    same queries 8 at a time (at most 64 workgroups each)."""
+    import torch
+    print(f"mq rounds {fmt} n={n} num_q={num_q} num_kv={num_kv} sub_n={sub_n}", flush=True)
+    make, call = _call(fmt)
+    rng = np.random.default_rng(n + sub_n)
+    kb, vb = _caches(rng, dev, fmt, n, num_kv)
+    qd = _dev(q_f16(rng, sub_n, num_q, 256).view(np.uint16), dev).view(torch.float16)
+    one, many = torch.zeros_like(qd), torch.zeros_like(qd)
+    ws = make(num_q, num_kv, sub_n, n, dev)
+    kw = dict(num_q=num_q, num_kv=num_kv, scale=1 / 16)
+    call(qd, kb, vb, one, ws, start_pos=n - sub_n, sub_n=sub_n, **kw)
+    torch.cuda.synchronize()
+    for t in range(0, sub_n, 8):
+        m = min(8, sub_n - t)
+        call(qd[t:t + m], kb, vb, many[t:t + m], ws, start_pos=n - sub_n + t, sub_n=m, **kw)
+    torch.cuda.synchronize()
+    one, many = one.float().cpu().numpy().reshape(sub_n, -1), many.float().cpu().numpy().reshape(sub_n, -1)
+    assert np.isfinite(many).all()
+    # Per query, 2-norms over all its heads: each path rounds its weights and its
+    # outputs to fp16 (2^-11 / sqrt(3) rms each), so two differ by about 1.15 x 2^-11.
+    # (rel_err's single elements are no measure over 8 million of them: the error of an
+    # outlier channel, 8 x the others', may fall in a row whose largest element is small.)
+    assert (np.linalg.norm(one - many, axis=1) / np.linalg.norm(many, axis=1)).max() < TOL
+
+
+@pytest.mark.parametrize("fmt", ["q8", "tq3"])
+def test_two_calls_on_two_streams(dev, fmt):
+    """Two verify calls of 256 workgroups each, one workgroup per CU, side by side
+    on two streams with workspaces of their own: neither may need all of its
+    workgroups to be resident."""
+    import torch
+    make, call = _call(fmt)
+    n, num_q, num_kv, sub_n = 32784, 16, 4, 16
+    rng = np.random.default_rng(9)
+    kb, vb = _caches(rng, dev, fmt, n, num_kv)
+    q = [_dev(q_f16(rng, sub_n, num_q, 256).view(np.uint16), dev).view(torch.float16) for _ in range(2)]
+    ws = [make(num_q, num_kv, sub_n, n, dev) for _ in range(2)]
+    kw = dict(num_q=num_q, num_kv=num_kv, start_pos=n - sub_n, sub_n=sub_n, scale=1 / 16)
+    want = [torch.zeros_like(x) for x in q]
+    for i in range(2):
+        call(q[i], kb, vb, want[i], ws[i], **kw)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = [[torch.zeros_like(x) for _ in range(8)] for x in q]
+    torch.cuda.synchronize()
+    for r in range(8):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                call(q[i], kb, vb, got[i][r], ws[i], **kw)
+    torch.cuda.synchronize()
+    for i in range(2):
+        for r in range(8):
+            assert torch.equal(got[i][r], want[i]), f"stream {i}, call {r}"

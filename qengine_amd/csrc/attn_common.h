@@ -367,6 +367,12 @@ hipError_t launch_q8_attn_fast_append(const AttnArgs& a, uint16_t* out, hipStrea
 hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* out, hipStream_t stream);
 // The merge of a launch's records as a launch of its own (attn_merge.hip); rotate: TQ3 values.
 hipError_t launch_record_merge(const AttnArgs& a, bool rotate, uint16_t* out, hipStream_t stream);
+// Whether a call's records are merged that way, and not by workgroups of the launch
+// that waits for them: with more merge units than half of the workgroups that the GPU
+// holds at once (`resident`), waiting workgroups could fill it, with two such launches
+// side by side or one of several rounds, while writers are still to run (100 paged
+// slots of 4 kv heads: 416 workgroups that all wait, on 256 CUs).
+inline bool merges_apart(const AttnArgs& a, long resident) { return 2L * a.num_q * a.sub_n > resident / 2; }
 hipError_t launch_mq_split(const AttnArgs& a, bool tq3, hipStream_t stream);
 hipError_t launch_split_merge(const float* m, const float* l, const float* o, uint16_t* out,
                               int num_q, int sub_n, int sub_n_max, int k_splits,

@@ -2,8 +2,9 @@
 // fast paths (TQ3 and Q8_0 caches).  Every workgroup of a launch writes one
 // record per (q head, query, key chunk) {m, l, o[256]}; the last workgroups of
 // the grid are designated mergers, one per (q head, query, 128-dim block)
-// unit, and turn the unit's records into the fp16 output.  attn_mq.hip
-// leaves that to a second launch instead (record_merge_kernel, attn_merge.hip).
+// unit, and turn the unit's records into the fp16 output.  Calls with many
+// units, and those of attn_mq.hip, leave that to a second launch instead
+// (record_merge_kernel, attn_merge.hip).
 //
 // Records move between workgroups (possibly on different XCDs, whose L2s are
 // not coherent with each other) with buffer accesses carrying the sc0|sc1
@@ -17,9 +18,10 @@
 // after this one on the stream, starts from, and the state of a zero-filled
 // workspace.  No counter or epoch is involved, and no workgroup pays an L2
 // write-back or invalidate (what agent-scope fences cost on this GPU).
-// Only mergers wait, after they have written their own records, and they are the
-// last workgroups of the grid: a launch whose merge units are fewer than its
-// workgroups never waits with all of them.  Their wait is bounded:
+// Only mergers wait.  They have written their own records by then, they are the
+// last workgroups of the grid, and they are at most half of those that the GPU
+// holds at once (merges_apart): the others never wait, and find room to run
+// also while another such launch is on the GPU.  Their wait is bounded:
 // a merger that runs out of polls writes NaN rows and sets the sticky error
 // word of the workspace header (one relaxed agent-scope store), which the host
 // reads with qkv_decode_workspace_status and clears with
@@ -285,14 +287,32 @@ __device__ bool merge_unit(float* red, f2_t* mls, const AttnArgs& p, __amdgpu_bu
   return true;
 }
 
+// Tag this workgroup's records (rows 0..rows-1 as in store_records) once every
+// thread's data stores are complete; every thread of the workgroup calls it.
+// gqa = num_q / num_kv, passed in uniform (scalar register).  apart: the records
+// are merged by the next launch, which waits for this one's stores by itself.
+__device__ __forceinline__ void publish_records(const AttnArgs& p, __amdgpu_buffer_rsrc_t rml, int h,
+                                                int gqa, int t0, int rows, int chunk, bool apart) {
+  if (!apart) {   // (uniform)
+    __builtin_amdgcn_s_waitcnt(0);  // this thread's data stores are complete
+    __syncthreads();
+  }
+  if ((int)threadIdx.x < rows) {
+    const int r = threadIdx.x;
+    __builtin_amdgcn_raw_buffer_store_b64(
+        u2_t{kTagValid, kTagValid}, rml,
+        (uint32_t)(rec_index(p, h * gqa + r % gqa, t0 + r / gqa, chunk) * kRecMlBytes + 8), 0, kCoherent);
+  }
+}
+
 // Store this workgroup's merged rows as records: row r = qi * gqa + hh (q head
 // h*gqa + hh of query t0 + qi) with data mo[r][256], maxima Mv[r] (log2
-// units) and sums Lv[r]; data first, then (once every thread's data stores
-// are complete) the tags of both 128-block units.
+// units) and sums Lv[r]; data first, then the tags of both 128-block units
+// (`apart`: a merge launch follows, as for publish_records).
 template <int THREADS>
 __device__ void store_records(const float* mo, const float* Mv, const float* Lv,
                               const AttnArgs& p, __amdgpu_buffer_rsrc_t rml,
-                              __amdgpu_buffer_rsrc_t ro, int h, int t0, int rows, int chunk) {
+                              __amdgpu_buffer_rsrc_t ro, int h, int t0, int rows, int chunk, bool apart) {
   constexpr int kHD = 256;
   const int gqa = p.num_q / p.num_kv;
   for (int idx = threadIdx.x; idx < rows * 64; idx += THREADS) {
@@ -304,14 +324,7 @@ __device__ void store_records(const float* mo, const float* Mv, const float* Lv,
       __builtin_amdgcn_raw_buffer_store_b64(f2_t{Mv[r], Lv[r]}, rml,
                                             (uint32_t)(rec * kRecMlBytes), 0, kCoherent);
   }
-  __builtin_amdgcn_s_waitcnt(0);  // this thread's data stores are complete
-  __syncthreads();
-  if ((int)threadIdx.x < rows) {
-    const int r = threadIdx.x;
-    __builtin_amdgcn_raw_buffer_store_b64(
-        u2_t{kTagValid, kTagValid}, rml,
-        (uint32_t)(rec_index(p, h * gqa + r % gqa, t0 + r / gqa, chunk) * kRecMlBytes + 8), 0, kCoherent);
-  }
+  publish_records(p, rml, h, gqa, t0, rows, chunk, apart);
 }
 
 // One 4-float piece of a record (row of q head qh, query t, chunk), written
@@ -324,21 +337,6 @@ __device__ __forceinline__ void store_record_piece(const AttnArgs& p, __amdgpu_b
   __builtin_amdgcn_raw_buffer_store_b128(o, ro, (uint32_t)((rec * 256 + d4) * 4), 0, kCoherent);
   if (d4 == 0)
     __builtin_amdgcn_raw_buffer_store_b64(f2_t{M, L}, rml, (uint32_t)(rec * kRecMlBytes), 0, kCoherent);
-}
-
-// Tag this workgroup's records (rows 0..rows-1 as in store_records) once every
-// thread's data stores are complete; every thread of the workgroup calls it.
-// gqa = num_q / num_kv, passed in uniform (scalar register).
-__device__ __forceinline__ void publish_records(const AttnArgs& p, __amdgpu_buffer_rsrc_t rml, int h,
-                                                int gqa, int t0, int rows, int chunk) {
-  __builtin_amdgcn_s_waitcnt(0);  // this thread's data stores are complete
-  __syncthreads();
-  if ((int)threadIdx.x < rows) {
-    const int r = threadIdx.x;
-    __builtin_amdgcn_raw_buffer_store_b64(
-        u2_t{kTagValid, kTagValid}, rml,
-        (uint32_t)(rec_index(p, h * gqa + r % gqa, t0 + r / gqa, chunk) * kRecMlBytes + 8), 0, kCoherent);
-  }
 }
 
 // The designated mergers: the last min(units, grid) workgroups merge the

@@ -7,6 +7,7 @@
 //
 // record_merge_kernel is the same merge over the records of a decode launch.
 #include <algorithm>
+#include <type_traits>
 
 #include "attn_common.h"
 #include "attn_fastmerge.h"
@@ -100,12 +101,11 @@ hipError_t launch_ws_status(const void* workspace, int* status, int ok_value, in
   return hipGetLastError();
 }
 
-// The records of a multi-query decode launch (attn_mq.hip), which precedes this one on
-// the stream, to the output: one workgroup per (query, q head, 128-dim block) unit.  A
-// launch of its own, because every workgroup of that one writes records that units all
-// over the grid need: workgroups that wait for records in the launch that writes them
-// hold the CUs that its other workgroups, or those of a launch on another stream, are
-// still to run on.  The records are complete
+// The records of a decode launch, which precedes this one on the stream, to the output:
+// one workgroup per (query, q head, 128-dim block) unit.  A launch of its own for calls
+// whose units are many (merges_apart) and for attn_mq.hip: workgroups that wait for
+// records in the launch that writes them hold the CUs that its other workgroups, or
+// those of a launch on another stream, are still to run on.  The records are complete
 // here, so their scalars and rows are loaded at once, one memory round trip; the
 // arguments are scalars that arrive in registers with the wave (attn_common.h) and the
 // unit comes from the three grid dimensions, without a division.
@@ -115,11 +115,45 @@ hipError_t launch_ws_status(const void* workspace, int* status, int ok_value, in
 // 8 queries over 301 keys 15.0 -> 13.0, 5 over 18,016 21.2 -> 20.0, 16 over 32,767
 // 36.4 -> 36.4; Q8_0, 16 over 4,096 19.1 -> 18.4, 2 over 18,016 20.9 -> 21.8.
 constexpr int kRecThreads = 256;
-template <bool ROTATE>
+
+// Sum over the wave, in every lane (the steps of wave_sum, attn_common.h).
+__device__ __forceinline__ int wave_sum_int(int v) {
+  auto add = [&](auto ctrl, auto rows) {
+    v += __builtin_amdgcn_update_dpp(0, v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+  };
+  using std::integral_constant;
+  add(integral_constant<int, 0xB1>{}, integral_constant<int, 0xf>{});    // quad_perm [1,0,3,2]
+  add(integral_constant<int, 0x4E>{}, integral_constant<int, 0xf>{});    // quad_perm [2,3,0,1]
+  add(integral_constant<int, 0x124>{}, integral_constant<int, 0xf>{});   // row_ror:4
+  add(integral_constant<int, 0x128>{}, integral_constant<int, 0xf>{});   // row_ror:8
+  add(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15
+  add(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});   // row_bcast:31
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// slot_shares (attn_fastmerge.h) by a wave: a slot per lane, one round of loads and of
+// divisions instead of one per slot.
+__device__ __forceinline__ void wave_slot_shares(const AttnArgs& p, int s, int& first, int& count) {
+  const int lane = threadIdx.x & 63;
+  long total = 0;
+  for (int i0 = 0; i0 < p.sub_n; i0 += 64) {
+    const int keys = i0 + lane < p.sub_n ? slot_keys(p, i0 + lane) : 0;
+    total += ((long)wave_sum_int(keys >> 16) << 16) + wave_sum_int(keys & 0xffff);
+  }
+  first = count = 0;
+  for (int i0 = 0; i0 <= s; i0 += 64) {
+    const int w = i0 + lane <= s ? share_count(p, i0 + lane, total) : 0;
+    first += wave_sum_int(i0 + lane < s ? w : 0);
+    if (s - i0 < 64) count = __builtin_amdgcn_readlane(w, s - i0);
+  }
+}
+
+template <bool ROTATE, bool RAGGED>
 __global__ __launch_bounds__(kRecThreads) void record_merge_kernel(float* ws_ml, float* ws_o, int* ws_header,
                                                                    uint16_t* out, uint32_t ws_ml_bytes,
                                                                    uint32_t ws_o_bytes, int num_q, int sub_n,
-                                                                   int n, int spin_limit) {
+                                                                   int n_chunks, int spin_limit,
+                                                                   const int32_t* ctx_lens, int ctx_max) {
   using ML = MergeLayout<kRecThreads>;
   __shared__ __attribute__((aligned(16))) float red[ML::kRedFloats];
   __shared__ f2_t mls[128];
@@ -127,10 +161,18 @@ __global__ __launch_bounds__(kRecThreads) void record_merge_kernel(float* ws_ml,
   AttnArgs p{};
   p.num_q = num_q;
   p.sub_n = sub_n;
-  p.n_slots = n;
+  p.n_slots = p.n_chunks = n_chunks;
   const int tid = threadIdx.x;
   const int t = blockIdx.x, qh = blockIdx.y, blk = blockIdx.z;
-  const long base = rec_index(p, qh, t, 0);
+  long base = rec_index(p, qh, t, 0);
+  int n = n_chunks;
+  if constexpr (RAGGED) {   // the slot's shares of the kv head's records
+    p.ctx_lens = ctx_lens;
+    p.ctx_max = ctx_max;
+    int first;
+    wave_slot_shares(p, t, first, n);
+    base = rec_index(p, qh, 0, first);
+  }
   const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(ws_ml, 0, ws_ml_bytes, kBufferRsrcWord3);
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(ws_o, 0, ws_o_bytes, kBufferRsrcWord3);
   const bool poisoned = __hip_atomic_load(ws_header + kWsErrorWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
@@ -165,9 +207,11 @@ __global__ __launch_bounds__(kRecThreads) void record_merge_kernel(float* ws_ml,
 
 hipError_t launch_record_merge(const AttnArgs& a, bool rotate, uint16_t* out, hipStream_t stream) {
   const dim3 grid(a.sub_n, a.num_q, 2), block(kRecThreads);
-  auto* kernel = rotate ? record_merge_kernel<true> : record_merge_kernel<false>;
+  auto* kernel = a.ctx_lens ? record_merge_kernel<true, true>   // (paged caches are TQ3)
+                 : rotate   ? record_merge_kernel<true, false>
+                            : record_merge_kernel<false, false>;
   hipLaunchKernelGGL(kernel, grid, block, 0, stream, a.ws_ml, a.ws_o, a.ws_header, out, a.ws_ml_bytes, a.ws_o_bytes,
-                     a.num_q, a.sub_n, a.n_chunks, a.spin_limit);
+                     a.num_q, a.sub_n, a.n_chunks, a.spin_limit, a.ctx_lens, a.ctx_max);
   return hipGetLastError();
 }
 

@@ -578,7 +578,8 @@ __global__ __launch_bounds__(kThreads, 2) void q8_attn_kernel(QKV_ATTN_LEAD_PARA
   const __amdgpu_buffer_rsrc_t ro =
       __builtin_amdgcn_make_buffer_rsrc(p.ws_o, 0, p.ws_o_bytes, kBufferRsrcWord3);
   if (has_work)
-    store_records<kThreads>(mo, ml + kMlM, ml + kMlL, p, rml, ro, h, t_idx, rows, split);
+    store_records<kThreads>(mo, ml + kMlM, ml + kMlL, p, rml, ro, h, t_idx, rows, split, out == nullptr);
+  if (out == nullptr) return;   // (merged by a launch of its own)
   merge_phase<kThreads, VTQ3>(reinterpret_cast<float*>(lds + kLdsMergeO),
                                reinterpret_cast<f2_t*>(lds + kLdsMergeML), p, rml, ro, out);
 }
@@ -591,34 +592,32 @@ hipError_t launch_q8_attn_split(const AttnArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// Workgroups of a fast-path launch: eight (query, chunk) groups of num_kv at a
-// time, and at least one workgroup per merge unit up to the 512 that reside at
-// once -- a short context with several queries has more units than chunks, and
-// a merger takes its units one after the other (8 queries over 301 keys: 256
-// units on 96 workgroups, 14.6 us; a workgroup each, 10.2).
-static int fast_grid(const AttnArgs& a) {
+// A fast-path launch: eight (query, chunk) groups of num_kv workgroups at a time, and
+// at least one workgroup per merge unit -- a short context with several queries has
+// more units than chunks, and a merger takes its units one after the other (8 queries
+// over 301 keys: 256 units on 96 workgroups, 14.6 us; a workgroup each, 10.2).
+constexpr int kResident = 512;   // workgroups that the GPU holds at once: two per CU
+template <class Kernel>
+static hipError_t launch_fast(Kernel kernel, const AttnArgs& a, bool v_tq3, uint16_t* out, hipStream_t stream) {
   const int per = 8 * a.num_kv;
-  const int groups = a.sub_n * a.n_chunks;
-  const int mergers = (int)std::min<long>(2L * a.num_q * a.sub_n, 512);
-  return std::max((groups + 7) / 8, (mergers + per - 1) / per) * per;
+  int n_wg = (a.sub_n * a.n_chunks + 7) / 8 * per;
+  const bool apart = merges_apart(a, kResident);
+  if (!apart) n_wg = std::max(n_wg, (2 * a.num_q * a.sub_n + per - 1) / per * per);
+  hipLaunchKernelGGL(kernel, dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, apart ? nullptr : out);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || !apart ? e : launch_record_merge(a, v_tq3, out, stream);
 }
 
 hipError_t launch_q8_attn_fast(const AttnArgs& a, uint16_t* out, hipStream_t stream) {
-  const int n_wg = fast_grid(a);
-  hipLaunchKernelGGL((q8_attn_kernel<0>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
-  return hipGetLastError();
+  return launch_fast(q8_attn_kernel<0>, a, false, out, stream);
 }
 
 hipError_t launch_q8_attn_fast_append(const AttnArgs& a, uint16_t* out, hipStream_t stream) {
-  const int n_wg = fast_grid(a);
-  hipLaunchKernelGGL((q8_attn_kernel<0, false, true>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
-  return hipGetLastError();
+  return launch_fast(q8_attn_kernel<0, false, true>, a, false, out, stream);
 }
 
 hipError_t launch_q8k_tq3v_attn_fast(const AttnArgs& a, uint16_t* out, hipStream_t stream) {
-  const int n_wg = fast_grid(a);
-  hipLaunchKernelGGL((q8_attn_kernel<0, true>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
-  return hipGetLastError();
+  return launch_fast(q8_attn_kernel<0, true>, a, true, out, stream);
 }
 
 }  // namespace qkv

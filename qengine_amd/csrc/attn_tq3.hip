@@ -1105,8 +1105,9 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
 
   // ---------------- fast path: tagged records, designated mergers ----------------
   QKV_STAMP(kPhMerged);
-  if (has_work) publish_records(p, rml, h, gqa_m, rec_t0, rows, rec_chunk);
+  if (has_work) publish_records(p, rml, h, gqa_m, rec_t0, rows, rec_chunk, out == nullptr);
   QKV_STAMP(kPhPublished);
+  if (out == nullptr) return;   // (merged by a launch of its own)
 #ifdef QKV_PHASE_TRACE
   if (threadIdx.x < 3) *reinterpret_cast<uint64_t*>(lds + kLdsMergeO + kTracePolledByte + 8 * threadIdx.x) = 0;
 #endif
@@ -1180,28 +1181,30 @@ hipError_t noalloc_scratch(int device, bool clear, hipStream_t stream, void** pt
   return hipSuccess;
 }
 
-constexpr int kMaxGrid = 256;   // workgroups that reside at once (one per CU)
+constexpr int kResident = 256;   // workgroups that the GPU holds at once: one per CU
 hipError_t launch_tq3_attn(const AttnArgs& a, int mode, uint16_t* out, hipStream_t stream) {
   const int groups = (a.sub_n + a.qpw - 1) / a.qpw * a.n_chunks;
   const int per = 8 * a.num_kv;
   int n_wg = (groups + 7) / 8 * per;
-  // Fast path: one workgroup per merge unit, up to one per CU -- a short context
-  // with several queries has more units than chunks, and a merger takes its
-  // units one after the other (4 queries over 301 keys: 128 units on 32
-  // workgroups 22.7 us, on 128 15.3).
-  if (mode == 0) n_wg = std::max(n_wg, ((int)std::min<long>(2L * a.num_q * a.sub_n, kMaxGrid) + per - 1) / per * per);
+  const bool apart = mode == 0 && merges_apart(a, kResident);
+  // Fast path: one workgroup per merge unit -- a short context with several queries
+  // has more units than chunks, and a merger takes its units one after the other
+  // (4 queries over 301 keys: 128 units on 32 workgroups 22.7 us, on 128 15.3).
+  if (mode == 0 && !apart) n_wg = std::max(n_wg, (2 * a.num_q * a.sub_n + per - 1) / per * per);
+  uint16_t* merged = apart ? nullptr : out;
   dim3 grid(n_wg), block(kThreads);
   if (mode == 0 && a.qpw * (a.num_q / a.num_kv) > 8)
-    hipLaunchKernelGGL((tq3_attn_kernel<0, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((tq3_attn_kernel<0, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, merged);
   else if (mode == 0 && a.k_new != nullptr)
-    hipLaunchKernelGGL((tq3_attn_kernel<0, false, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((tq3_attn_kernel<0, false, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, merged);
   else if (mode == 0)
-    hipLaunchKernelGGL((tq3_attn_kernel<0>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
+    hipLaunchKernelGGL((tq3_attn_kernel<0>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, merged);
   else if (mode == 1)
     hipLaunchKernelGGL((tq3_attn_kernel<1>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
   else
     hipLaunchKernelGGL((tq3_attn_kernel<2>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a, out);
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || !apart ? e : launch_record_merge(a, true, out, stream);
 }
 
 }  // namespace qkv

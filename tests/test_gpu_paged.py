@@ -130,6 +130,36 @@ def test_ragged_shared_prefix_vs_oracle(dev, block_tokens, num_q):
         assert_tq3_attn(got[s], exp[s], ex[s], what=s)
 
 
+@pytest.mark.parametrize("num_q,num_kv,n_slots", [
+    (16, 4, 100),    # 400 workgroups with work on 256 CUs
+    (8, 1, 100),     # 200: record shares left over to hand out, in two runs of 64 slots
+    (16, 4, 5),      # the first slot count whose records a second launch merges
+])
+def test_many_slots(dev, num_q, num_kv, n_slots):
+    """More slots than a round of the GPU holds (no workgroup may wait for one that
+    has no CU yet), contexts of 0 to 700 keys.  Per slot, 2-norm over its heads:
+    fp16 weights and outputs (2^-11 / sqrt(3) rms each) are 3.4e-4 beside the exact
+    attention; three times that is the bar."""
+    rng = np.random.default_rng(n_slots + num_kv)
+    bt_tok = 64
+    ctx = rng.integers(0, 701, size=n_slots)
+    ctx[0], ctx[-1] = 700, 1
+    max_ctx = int(ctx.max())
+    max_blocks = (max_ctx + bt_tok - 1) // bt_tok
+    n_phys = int(sum((c + bt_tok - 1) // bt_tok for c in ctx))
+    bt = _tables(rng, ctx, bt_tok, max_blocks, n_phys)
+    kp, vp = _pool(rng, n_phys * bt_tok, num_kv)
+    q = q_f16(rng, n_slots, num_q, HD)
+    print(f"paged n_slots={n_slots} num_q={num_q} num_kv={num_kv}", flush=True)
+    got = _decode(dev, q, kp, vp, bt, ctx, num_q=num_q, num_kv=num_kv, max_ctx=max_ctx,
+                  block_tokens=bt_tok).astype(np.float64).reshape(n_slots, -1)
+    ex = _exact_paged(q, kp, vp, bt, ctx, num_q=num_q, num_kv=num_kv,
+                      block_tokens=bt_tok).reshape(n_slots, -1)
+    assert np.all(got[ctx == 0] == 0)
+    live = ctx > 0
+    assert (np.linalg.norm(got - ex, axis=1)[live] / np.linalg.norm(ex, axis=1)[live]).max() < 1e-3
+
+
 def test_zero_and_clamped_context(dev):
     """ctx 0 gives a zero row; ctx beyond max_ctx is clamped to max_ctx."""
     rng = np.random.default_rng(5)

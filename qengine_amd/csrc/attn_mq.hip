@@ -21,7 +21,13 @@
 //            probabilities go to LDS as fp16 in the operand order of the value
 //            product.  A score above the reference by more than kSlack (the
 //            first tile, rarely later) raises it: only then do the key groups
-//            exchange maxima and the sums and accumulators get rescaled.
+//            exchange maxima and the sums and accumulators get rescaled.  The
+//            largest weight is therefore not 1 and exact, but rounded like the
+//            others: with Q8_0 values (whose weights carry no norm to round) what
+//            the rounding leaves out is kept as a second fp16 number, with a
+//            product of its own, so that the rows are no further from the exact
+//            ones than with a running maximum in every wave (2-norm, 16 queries
+//            over 4,096 keys: 6.30e-4 there, 6.48e-4 with one product).
 //   values   wave w owns dims 32 w .. 32 w + 31 of all columns: A = the
 //            probabilities (one 16-byte read per 16 columns and 32 keys), B =
 //            its own dims of 32 keys, decoded in registers.  32 accumulators
@@ -80,7 +86,8 @@ struct MqLds {
   // piece c at c ^ ((r >> 1) & 7) (16 rows at one logical piece: 16 bank groups)
   static constexpr int kKBuf = KT ? kTile * 128 : kTile * kQ8Pitch;
   static constexpr int kVBuf = VT ? 32 * kVgPitch * 4 : kTile * kQ8Pitch;
-  static constexpr int kPBuf = (VT ? 2 : 1) * 64 * 128;   // [64 columns][64 keys] fp16 (TQ3: per 128-block)
+  // [64 columns][64 keys] fp16: TQ3 values one per 128-block, Q8_0 values the weights and their rests
+  static constexpr int kPBuf = 2 * 64 * 128;
   static constexpr int kK = VT ? kLutBytes : 0;           // three buffers each
   static constexpr int kV = kK + 3 * kKBuf;
   // TQ3 norms [3 buffers][keys block 0, 1 (x the softmax scale), values block 0, 1][64] f32
@@ -651,10 +658,14 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
             *reinterpret_cast<h4_t*>(pd + 2048 * cg + j * 64 * 128) = w;
           }
         } else {
-          h4_t w;
+          h4_t w, rest;
 #pragma unroll
-          for (int r = 0; r < 4; r++) w[r] = (_Float16)pr[r];
+          for (int r = 0; r < 4; r++) {
+            w[r] = (_Float16)pr[r];
+            rest[r] = (_Float16)(pr[r] - (float)w[r]);
+          }
           *reinterpret_cast<h4_t*>(pd + 2048 * cg) = w;
+          *reinterpret_cast<h4_t*>(pd + 64 * 128 + 2048 * cg) = rest;
         }
       }
       return top;
@@ -726,8 +737,8 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     }
     // ---- values: acc[g][e] += P(16 columns x 32 keys) V(32 keys x 16 dims)
     const uint8_t* pbase = pbuf + (VT ? (wave >> 2) * 64 * 128 : 0);
-    auto p_operand = [&](int g, int c2) {   // columns 16 g + n, keys of half c2
-      return *reinterpret_cast<const h8_t*>(pbase + 16 * g * 128 + (p_at ^ (64 * c2)));
+    auto p_operand = [&](int g, int c2, int rest = 0) {   // columns 16 g + n, keys of half c2
+      return *reinterpret_cast<const h8_t*>(pbase + rest * 64 * 128 + 16 * g * 128 + (p_at ^ (64 * c2)));
     };
     // B operands of half c2: dims 32 wave + 2 n (bv[0]) and + 1 (bv[1])
     auto v_operands = [&](int c2, u4_t (&bv)[2]) {
@@ -794,14 +805,20 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       for (int c2 = 0; c2 < 2; c2++) {
         u4_t bv[2];
         v_operands(c2, bv);
-        h8_t pa[NG];
+        auto product = [&](int rest) {
+          h8_t pa[NG];
 #pragma unroll
-        for (int g = 0; g < NG; g++) pa[g] = p_operand(g, c2);
+          for (int g = 0; g < NG; g++) pa[g] = p_operand(g, c2, rest);
 #pragma unroll
-        for (int g = 0; g < NG; g++)
+          for (int g = 0; g < NG; g++)
 #pragma unroll
-          for (int e = 0; e < 2; e++)
-            acc[g][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g], __builtin_bit_cast(h8_t, bv[e]), acc[g][e], 0, 0, 0);
+            for (int e = 0; e < 2; e++)
+              acc[g][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g], __builtin_bit_cast(h8_t, bv[e]), acc[g][e], 0, 0, 0);
+        };
+        product(0);
+        // (with an inf scale the weights' rests, 0 among them, would make NaN of inf)
+        if constexpr (!VT)
+          if (!v_nonfinite) product(1);
       }
     }
     const int b = b0;

@@ -325,9 +325,11 @@ static int tq3_split_mq(int gqa, int num_kv, int sub_n, int k_splits, int m) {
 // Q8_0: one query per workgroup against every query that 32 columns hold (64 where 32
 // would take several rounds).  One workgroup alone reads its split at the rate of a
 // CU's memory pipe, and so does a pair on one CU together: the multi-query kernel wins
-// once the queries no longer spread over idle CUs.  18,016 keys in 8 splits, 16 queries:
-// 95 -> 71 us, 8 queries (256 workgroups): 64, not 71; 32 splits, 16 queries: 97 -> 26.
-// Splits of a tile or two: 9.9, not 10.4, with 512 workgroups, 13.7 -> 11.8 with 1,024.
+// once the queries no longer spread over idle CUs.  With the merge call, us: 18,016 keys
+// in 8 splits, 16 queries 91 -> 77, 8 queries (256 workgroups) 59, not 77; in 32 splits,
+// 16 queries 108 -> 37; 5,000 keys in 8 splits, 9 queries 32.4 -> 27.9.  Splits of a tile
+// or two are level up to 512 workgroups (8 queries over 900 keys in 16 splits 13.5, not
+// 14.6; 4 over 2,000 in 32 18.5, not 17.7), past that 8 over 2,000 take 20.1, not 26.4.
 static int q8_split_mq(int gqa, int num_kv, int sub_n, int k_splits, int m) {
   const long old_wgs = (long)num_kv * k_splits * sub_n;
   if (sub_n == 1 || old_wgs <= (m < 192 ? 512 : 256)) return 0;

@@ -169,3 +169,49 @@ def test_two_calls_on_two_streams(dev, fmt):
     for i in range(2):
         for r in range(8):
             assert torch.equal(got[i][r], want[i]), f"stream {i}, call {r}"
+
+
+def _exact_q8(rng, n, num_kv):
+    """Q8_0 rows whose scales are powers of two, so that their fp16 values are
+    exact: (blocks, values float64 [n][num_kv][256])."""
+    code = rng.integers(-127, 128, size=(n, num_kv, 8, 32)).astype(np.int8)
+    scale = (2.0 ** -rng.integers(5, 9, size=(n, num_kv, 8))).astype(np.float16)
+    b = np.zeros((n, num_kv, 8, 36), np.uint8)
+    b[..., :32] = code.view(np.uint8)
+    b[..., 34:] = scale[..., None].view(np.uint8)
+    return b, (code * scale[..., None].astype(np.float64)).reshape(n, num_kv, 256)
+
+
+@pytest.mark.parametrize("sub_n,num_q,num_kv", [(6, 16, 4), (16, 16, 4), (9, 24, 4)])
+def test_weights_keep_more_than_fp16(dev, sub_n, num_q, num_kv):
+    """Over caches whose decoded values are exact only the weights are left to round.
+    Their fp16 roundings alone would be 2^-12 of a row; with their rests in a product
+    of their own what remains is the fp32 sums (2,000 terms, about 2^-20), so the
+    split API's rows are held to 2^-15 and all but the ties among the decode's fp16
+    rows are the exact ones rounded (error 2^-20 against a spacing of at least 2^-11:
+    1 in 500 lies across; with rounded weights every third did)."""
+    import torch
+    from qengine_amd import kvcache
+    n, ks, gqa = 2000, 32, num_q // num_kv
+    rng = np.random.default_rng(sub_n + num_q)
+    (kb, k), (vb, v) = _exact_q8(rng, n, num_kv), _exact_q8(rng, n, num_kv)
+    q = (q_f16(rng, sub_n, num_q, 256).astype(np.float32) * 0.4).astype(np.float16)
+    s = np.einsum("tqd,nqd->tqn", q.astype(np.float64), np.repeat(k, gqa, 1)) / 16
+    s = np.where(np.arange(n) > n - sub_n + np.arange(sub_n)[:, None, None], -np.inf, s)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    vq = np.repeat(v, gqa, 1)
+    want = np.einsum("tqn,nqd->tqd", p / p.sum(-1, keepdims=True), vq)
+    kd, vd, qd = _dev(kb, dev), _dev(vb, dev), _dev(q.view(np.uint16), dev).view(torch.float16)
+    kw = dict(num_q=num_q, num_kv=num_kv, start_pos=n - sub_n, sub_n=sub_n, scale=1 / 16)
+    out = torch.zeros_like(qd)
+    kvcache.decode_attn_q8(qd, kd, vd, out, kvcache.decode_attn_q8_workspace(num_q, num_kv, sub_n, n, dev), **kw)
+    pm, pl = (torch.zeros((num_q, sub_n, ks), device=dev) for _ in range(2))
+    po = torch.zeros((num_q, sub_n, ks, 256), device=dev)
+    kvcache.attn_split_q8(qd, kd, vd, pm, pl, po, sub_n_max=sub_n, active_end_max=n, k_splits=ks, **kw)
+    torch.cuda.synchronize()
+    differ = np.mean(out.cpu().numpy().view(np.uint16) != want.astype(np.float16).view(np.uint16))
+    assert differ < 0.01, differ
+    pm, pl, po = (x.cpu().numpy().astype(np.float64) for x in (pm, pl, po))
+    w = np.exp(pm - pm.max(-1, keepdims=True))
+    got = np.einsum("qtz,qtzd->tqd", w / (w * pl).sum(-1, keepdims=True), po)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 2.0 ** -15

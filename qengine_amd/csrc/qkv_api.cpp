@@ -698,10 +698,12 @@ int mq_geom(FastGeom& g, int num_q, int num_kv, int sub_n, int n_keys, int max_c
   return best_qpw;
 }
 
-// Most chunks of a TQ3 launch of that kernel over n_keys keys (monotone in n_keys).
-int mq_tq3_chunks(int num_kv, int n_keys) {
-  const int tiles = (n_keys + 63) / 64;
-  return std::min({128, (tiles + 1) / 2, std::max(1, (int)kMaxFastWgs / num_kv)});
+// Most chunks that mq_geom gives a TQ3 call over n_keys keys (monotone in n_keys): two
+// tiles each, and one round of workgroups with the fewest query groups.
+int mq_tq3_chunks(int num_q, int num_kv, int sub_n, int n_keys) {
+  const int tiles = (n_keys + 63) / 64, most = std::max(1, 64 / std::max(1, num_q / num_kv));
+  const long groups = (sub_n + most - 1) / most;
+  return (int)std::min<long>({128, (tiles + 1) / 2, std::max(1l, kMaxFastWgs / (groups * num_kv))});
 }
 bool tq3_takes_mq(int num_q, int num_kv, int sub_n) { return (long)sub_n * (num_q / num_kv) > 16; }
 }  // namespace
@@ -712,7 +714,7 @@ size_t qkv_decode_attn_tq3_workspace_bytes(int num_q, int num_kv, int sub_n, int
                              tq3_join_min(num_q, num_kv, sub_n));
   if (tq3_takes_mq(num_q, num_kv, sub_n)) {
     FastGeom g{};
-    g.n_chunks = mq_tq3_chunks(num_kv, n_keys);
+    g.n_chunks = mq_tq3_chunks(num_q, num_kv, sub_n, n_keys);
     set_layout(g, num_q, sub_n);
     need = std::max(need, g.total);
   }
@@ -739,10 +741,11 @@ static int decode_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block
   const bool mq = tq3_takes_mq(num_q, num_kv, sub_n);
   if (mq) {
     FastGeom m = g;
-    const int mqpw = mq_geom(m, num_q, num_kv, sub_n, n_keys, mq_tq3_chunks(num_kv, n_keys));
+    const int mqpw = mq_geom(m, num_q, num_kv, sub_n, n_keys, mq_tq3_chunks(num_q, num_kv, sub_n, n_keys));
     set_layout(m, num_q, sub_n);
-    // (the fixed scratch of the allocation-free call may only hold the longer chunks)
-    if (!noalloc || m.total <= qkv::kNoAllocScratchBytes) {
+    // (the allocation-free call's fixed scratch, or a workspace sized for the longer
+    // chunks, may hold only those)
+    if (m.total <= std::min<size_t>(noalloc ? qkv::kNoAllocScratchBytes : workspace_bytes, 0xffffffffu)) {
       g = m;
       qpw = mqpw;
     }

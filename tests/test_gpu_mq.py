@@ -215,3 +215,34 @@ def test_weights_keep_more_than_fp16(dev, sub_n, num_q, num_kv):
     w = np.exp(pm - pm.max(-1, keepdims=True))
     got = np.einsum("qtz,qtzd->tqd", w / (w * pl).sum(-1, keepdims=True), po)
     assert np.linalg.norm(got - want) / np.linalg.norm(want) < 2.0 ** -15
+
+
+@pytest.mark.parametrize("sub_n", [16, 7])
+def test_tq3_workspace_of_the_longer_chunks(dev, sub_n):
+    """A workspace that holds one record per 512 keys, which is what a TQ3 call of
+    many queries needs at least, serves it with chunks of that length; so does the
+    8 MiB scratch of the allocation-free call, too small for the shorter chunks of 16
+    queries over 4,096 keys.  One byte less is refused."""
+    import torch
+    from qengine_amd import kvcache
+    n, num_q, num_kv, chunks = 4096, 16, 4, 8
+    rng = np.random.default_rng(sub_n)
+    kb, vb = _caches(rng, dev, "tq3", n, num_kv)
+    qd = _dev(q_f16(rng, sub_n, num_q, 256).view(np.uint16), dev).view(torch.float16)
+    kw = dict(num_q=num_q, num_kv=num_kv, start_pos=n - sub_n, sub_n=sub_n, scale=1 / 16)
+    rows = num_q * sub_n * chunks
+    need = (256 + 16 * rows + 255) // 256 * 256 + 1024 * rows
+    full_ws = kvcache.decode_attn_tq3_workspace(num_q, num_kv, sub_n, n, dev)
+    assert need < full_ws.numel() * full_ws.element_size()
+    full, small, noalloc = (torch.zeros_like(qd) for _ in range(3))
+    kvcache.decode_attn_tq3(qd, kb, vb, full, full_ws, **kw)
+    kvcache.decode_attn_tq3(qd, kb, vb, small, torch.zeros(need, dtype=torch.uint8, device=dev), **kw)
+    kvcache.decode_attn_tq3_noalloc(qd, kb, vb, noalloc, **kw)
+    torch.cuda.synchronize()
+    assert rel_err(full.float().cpu().numpy(), small.float().cpu().numpy()) < TOL
+    if sub_n == 16:
+        assert torch.equal(noalloc, small)
+    else:   # (the shorter chunks fit the scratch)
+        assert torch.equal(noalloc, full)
+    with pytest.raises(Exception):
+        kvcache.decode_attn_tq3(qd, kb, vb, small, torch.zeros(need - 1, dtype=torch.uint8, device=dev), **kw)

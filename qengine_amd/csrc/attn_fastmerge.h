@@ -88,13 +88,16 @@ __device__ inline int share_slot(const AttnArgs& p, int g, int& first, int& coun
 
 // Merger thread layout for a THREADS-thread workgroup: slices of 32 threads
 // (one dim quad of a 128-block each), 128/slices records per thread
-// (n_chunks <= 128).  The reduction area holds one 128-float partial per wave.
+// (n_chunks <= 128).  The reduction area holds one 128-float partial per wave,
+// then the vote's word per wave (not within the partials: a wave may fold while
+// another has still to read the vote).
 template <int THREADS>
 struct MergeLayout {
   static constexpr int kSlices = THREADS / 32;
   static constexpr int kRecPerThread = 128 / kSlices;
   static constexpr int kWaves = THREADS / 64;
-  static constexpr int kRedFloats = kWaves * 128;
+  static constexpr int kVote = kWaves * 128;
+  static constexpr int kRedFloats = kVote + kWaves;
 };
 
 // Workgroup-wide AND of `pred` over a 1-D workgroup of THREADS threads: one
@@ -242,8 +245,7 @@ __device__ bool merge_unit(float* red, f2_t* mls, const AttnArgs& p, __amdgpu_bu
         mls[tid] = f2_t{r[0], r[1]};
       }
     }
-    // (red is free until the rows are folded: it holds the vote)
-    if (block_and<THREADS>(seen, reinterpret_cast<int*>(red))) {
+    if (block_and<THREADS>(seen, reinterpret_cast<int*>(red + ML::kVote))) {
       complete = true;
       break;
     }

@@ -157,7 +157,6 @@ __global__ __launch_bounds__(kRecThreads) void record_merge_kernel(float* ws_ml,
   using ML = MergeLayout<kRecThreads>;
   __shared__ __attribute__((aligned(16))) float red[ML::kRedFloats];
   __shared__ f2_t mls[128];
-  __shared__ int vote[ML::kWaves];
   AttnArgs p{};
   p.num_q = num_q;
   p.sub_n = sub_n;
@@ -196,7 +195,7 @@ __global__ __launch_bounds__(kRecThreads) void record_merge_kernel(float* ws_ml,
   if (seen)   // clear: the state that the next launch on this workspace starts from
     __builtin_amdgcn_raw_buffer_store_b32(0u, rml, (uint32_t)((base + tid) * kRecMlBytes + 8 + 4 * blk), 0,
                                           kCoherent);
-  if (!block_and<kRecThreads>(seen || tid >= n, vote)) {
+  if (!block_and<kRecThreads>(seen || tid >= n, reinterpret_cast<int*>(red + ML::kVote))) {
     write_nan_unit(p, t, qh, blk, out);
     if (tid == 0)
       __hip_atomic_store(ws_header + kWsErrorWord, kWsErrorTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

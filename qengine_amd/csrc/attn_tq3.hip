@@ -884,10 +884,15 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
 
     if constexpr (first) QKV_STAMP(kPhScores);
     // ---------------- staging: value codes and norms ----------------
-    if constexpr (kUnits)
+    if constexpr (kUnits) {
+      // (they take the place of the key units, which other lanes have read)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       stage_values(st, lane_o, tr.v);
-    else
+    } else {
       stage_rows(st, lane_o, tr, scale2);
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");

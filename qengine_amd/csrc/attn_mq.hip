@@ -458,11 +458,14 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       }
     __syncthreads();   // the query scratch is read: the staging buffers are free
   }
-  // tiles before this key are seen whole by every column (the sink / window rule
-  // applies to every tile, the tree bits to keys past start_pos)
-  const int dense_end = KT && (p.sink_tok > 0 || p.window_tok > 0) ? 0
-                        : KT && p.tree_mask != nullptr             ? min(hi_first, p.start_pos)
-                                                                   : hi_first;
+  // tiles before this key are seen whole by every column, as far as the end of its keys
+  // and the tree bits (keys past start_pos) go
+  const int dense_end = KT && p.tree_mask != nullptr ? min(hi_first, p.start_pos) : hi_first;
+  // the sink / window rule on 32-key tiles (KeyRule), for all columns: seen by every one
+  // that has the whole tile among its keys, seen by none
+  const bool sw = KT && (p.sink_tok > 0 || p.window_tok > 0);
+  auto sw_all = [&](int t32) { return t32 < p.sink_tok || t32 + 32 > active_last - p.window_tok; };
+  auto sw_none = [&](int t32) { return t32 >= p.sink_tok && t32 + 32 <= p.start_pos + t0 + 1 - p.window_tok; };
   // (opaque thread indexes: the offsets of staging and loads are formed at each
   // use instead of being held in registers through the loop)
   auto stage = [&](int ts, int buf, MqRegs<KT, VT>& r) {
@@ -511,13 +514,36 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   // tile t's staging buffer and flag, those of t + 1 and of t + 2
   int b0 = 0, b1 = 1, b2 = 2;
   float slack = kSlack<VT>;
+  // behind a tile's barrier: tile t + 2 into the free buffer, t + 3 on its way
+  auto advance = [&](int ts, int t, int b2, MqRegs<KT, VT>& r) {
+    if constexpr (VT) slack = __builtin_amdgcn_readfirstlane(flag_s[3]) ? 0.0f : kSlack<VT>;
+    if (t + 2 < n_tiles) {
+      stage(ts + 2 * kTile, b2, r);
+      if (t + 3 < n_tiles) load(ts + 3 * kTile, r);
+    }
+    if (tid == 0) flag_s[b2] = 0;   // (set by tile t + 2, after the next barrier)
+  };
   for (int t = 0; t < n_tiles; t++) {
     const int ts = lo + t * kTile;
     const uint8_t* kbuf = lds + L::kK + b0 * L::kKBuf;
     const uint8_t* vbuf = lds + L::kV + b0 * L::kVBuf;
     const float* knorm = reinterpret_cast<const float*>(lds + L::kNorm) + b0 * 4 * kTile;
     uint8_t* pbuf = lds + L::kP + (t & 1) * L::kPBuf;
-    const bool dense = ts + kTile <= dense_end;
+    bool dense = ts + kTile <= dense_end;
+    if constexpr (KT) {
+      if (sw) {
+        dense = dense && sw_all(ts) && sw_all(ts + 32);
+        if (sw_none(ts) && sw_none(ts + 32)) {   // nothing of it counts: only keep the pipeline going
+          __syncthreads();
+          advance(ts, t, b2, ra);
+          const int b = b0;
+          b0 = b1;
+          b1 = b2;
+          b2 = b;
+          continue;
+        }
+      }
+    }
     bool v_nonfinite = false;
     if constexpr (!VT) {
       // the scales of this wave's value block, one key per lane, to the wave's own area
@@ -724,12 +750,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
           for (int r = 0; r < 4; r++) acc[g][e][r] *= cr[r];
       }
     }
-    if constexpr (VT) slack = __builtin_amdgcn_readfirstlane(flag_s[3]) ? 0.0f : kSlack<VT>;
-    if (t + 2 < n_tiles) {
-      stage(ts + 2 * kTile, b2, ra);
-      if (t + 3 < n_tiles) load(ts + 3 * kTile, ra);
-    }
-    if (tid == 0) flag_s[b2] = 0;   // (set by tile t + 2, after the next barrier)
+    advance(ts, t, b2, ra);
 #pragma unroll
     for (int cg = 0; cg < kCg; cg++) {
       lsum[cg] += ps[cg];

@@ -246,3 +246,34 @@ def test_tq3_workspace_of_the_longer_chunks(dev, sub_n):
         assert torch.equal(noalloc, full)
     with pytest.raises(Exception):
         kvcache.decode_attn_tq3(qd, kb, vb, small, torch.zeros(need - 1, dtype=torch.uint8, device=dev), **kw)
+
+
+@pytest.mark.parametrize("sink,window", [(0, 100), (64, 0), (33, 1000), (70, 64), (1, 3000), (4, 1 << 20), (5000, 1)])
+@pytest.mark.parametrize("sub_n,num_q", [(16, 16), (7, 16), (5, 24)])
+def test_tq3_sink_and_window(dev, sub_n, num_q, sink, window):
+    """Tiles that the sink / window rule shows whole to every query of a block, to
+    none of them (their rows, with an inf norm among them, are left out), and to
+    some, against the same queries one at a time (over rows without the inf)."""
+    import torch
+    from qengine_amd import kvcache
+    n, num_kv = 4300, 4
+    rng = np.random.default_rng(sink + window + sub_n)
+    k16, v16 = kv_f16(rng, n, num_kv, 256), kv_f16(rng, n, num_kv, 256)
+    kb, vb = O.tq3_encode(k16).view(np.uint8).reshape(n, -1), O.tq3_encode(v16).view(np.uint8).reshape(n, -1)
+    end = n - sub_n + 1
+    unseen = [r for r in range(end) if not any(
+        r // 32 * 32 < sink or min(r // 32 * 32 + 32, e) > e - window for e in range(end, n + 1))]
+    clean = _dev(vb.copy(), dev)
+    for r in unseen[::97]:
+        vb[r, :4] = np.frombuffer(np.float32(np.inf).tobytes(), np.uint8)
+    kd, vd = _dev(kb, dev), _dev(vb, dev)
+    qd = _dev(q_f16(rng, sub_n, num_q, 256).view(np.uint16), dev).view(torch.float16)
+    one, many = torch.zeros_like(qd), torch.zeros_like(qd)
+    ws = kvcache.decode_attn_tq3_workspace(num_q, num_kv, sub_n, n, dev)
+    kw = dict(num_q=num_q, num_kv=num_kv, scale=1 / 16, sink_tok=sink, window_tok=window)
+    kvcache.decode_attn_tq3(qd, kd, vd, one, ws, start_pos=n - sub_n, sub_n=sub_n, **kw)
+    for t in range(sub_n):
+        kvcache.decode_attn_tq3(qd[t:t + 1].contiguous(), kd, clean, many[t:t + 1], ws, start_pos=n - sub_n + t, sub_n=1, **kw)
+    torch.cuda.synchronize()
+    one, many = one.float().cpu().numpy(), many.float().cpu().numpy()
+    assert np.isfinite(many).all() and rel_err(one, many) < TOL

@@ -856,7 +856,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   // wave its dims of every column
   __syncthreads();
   float* sums = reinterpret_cast<float*>(lds + L::kSum);
-  int* recs = reinterpret_cast<int*>(lds + L::kSum + 5 * 64 * 4);
+  uint32_t* recs = reinterpret_cast<uint32_t*>(lds + L::kSum + 5 * 64 * 4);   // (byte offsets up to 4 GiB)
   const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(p.ws_ml, 0, p.ws_ml_bytes, kBufferRsrcWord3);
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(p.ws_o, 0, p.ws_o_bytes, kBufferRsrcWord3);
   int gqa_m = gqa;
@@ -933,7 +933,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     }
     return;
   }
-  if (tid_e < 64) recs[tid_e] = (int)rec_index(p, h * gqa_m + tid_e % gqa_m, t0 + min(tid_e, cols - 1) / gqa_m, chunk);
+  if (tid_e < 64) recs[tid_e] = (uint32_t)rec_index(p, h * gqa_m + tid_e % gqa_m, t0 + min(tid_e, cols - 1) / gqa_m, chunk);
   __syncthreads();
 #pragma unroll
   for (int g = 0; g < NG; g++) {
@@ -942,14 +942,14 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       const int R = 16 * g + 4 * kb_e + r;
       if (R < cols)
         __builtin_amdgcn_raw_buffer_store_b64(f2_t{acc[g][0][r], acc[g][1][r]}, ro,
-                                              (uint32_t)((recs[R] * kHD + 32 * wave + 2 * n_e) * 4), 0, kCoherent);
+                                              (recs[R] * kHD + (uint32_t)(32 * wave + 2 * n_e)) * 4u, 0, kCoherent);
     }
   }
   if (tid_e < cols) {
     const float l = (sums[tid_e] + sums[64 + tid_e]) + (sums[128 + tid_e] + sums[192 + tid_e]);
     __builtin_amdgcn_raw_buffer_store_b128(
         u4_t{__float_as_uint(sums[4 * 64 + tid_e]), __float_as_uint(l), kTagValid, kTagValid}, rml,
-        (uint32_t)(recs[tid_e] * kRecMlBytes), 0, kCoherent);
+        recs[tid_e] * kRecMlBytes, 0, kCoherent);
   }
 }
 

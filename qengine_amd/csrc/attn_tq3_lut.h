@@ -16,20 +16,6 @@ namespace qkv {
 constexpr int kLdsLut = 0;
 constexpr int kLdsLutBytes = 256 * 64 * 4;
 
-// The table's entries from immediates (wave-uniform values): wave w of 8 writes
-// every lane's copy of entries 32w .. 32w+31, (centroid[e & 7], centroid[(e >> 3) & 7]).
-__device__ __forceinline__ void tq3_lut_build(uint8_t* lds, int wave, uint32_t lane4) {
-  const uint32_t w = (uint32_t)wave;
-#pragma unroll
-  for (int hk = 0; hk < 4; hk++) {
-    const uint32_t hi = centroid_scaled_h((4u * w + hk) & 7u) << 16;
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      *reinterpret_cast<uint32_t*>(lds + kLdsLut + (w * 32 + hk * 8 + k) * 256 + lane4) =
-          centroid_scaled_h(k) | hi;
-  }
-}
-
 __device__ __forceinline__ uint32_t lut_read(const uint8_t* lds, uint32_t addr) {
   return *reinterpret_cast<const uint32_t*>(lds + kLdsLut + addr);
 }

@@ -136,9 +136,8 @@ def test_fast_decode_vs_oracle(dev, n, num_q, sub_n):
     (3000, 16, 20, 0, 0, False), (2500, 24, 16, 0, 0, True), (1800, 8, 33, 0, 0, False),
     # chunks grown to keep one round of workgroups: 2 and 3 tiles per wave
     (40000, 16, 1, 0, 0, False), (70000, 24, 1, 0, 0, False), (40000, 16, 2, 128, 2048, True),
-    # 16 queries x GQA 4 = 64 columns, every tile decoded once (tq3_mq_kernel):
-    # 64 chunks of 512 keys, the last also taking the remainder past 32768
-    # keys (16, 32 and 64 keys: joined; 65 keys: 33 chunks of 1024)
+    # 16 queries x GQA 4 = 64 columns, every tile read once (mq_attn_kernel), 513 or
+    # 514 tiles: the last one of 16, 32 or 64 keys, or one of 64 and one of a key
     (32784, 16, 16, 0, 0, False),
     (32800, 16, 16, 0, 0, False), (32832, 16, 16, 0, 0, True), (32833, 16, 16, 0, 0, False)])
 def test_fast_decode_multi_query(dev, n, num_q, sub_n, sink, window, tree):
@@ -146,8 +145,8 @@ def test_fast_decode_multi_query(dev, n, num_q, sub_n, sink, window, tree):
     last groups, GQA 1 to 8, causal, tree and sink/window masks; calls
     with at most 8 / GQA queries carry rounded query and remainder in one
     product, up to 16 / GQA queries the remainders ride in a chained product,
-    and calls with more than 16 (query, head) columns decode each tile once
-    for up to 64 of them (tq3_mq_kernel; GQA 4 x 16 queries, GQA 2 x 11,
+    and calls with more than 16 (query, head) columns read each tile once
+    for up to 64 of them (mq_attn_kernel; GQA 4 x 16 queries, GQA 2 x 11,
     GQA 1 x 17, GQA 8 x 3, partial column groups, several query blocks)."""
     from qengine_amd import kvcache
     torch = _torch()

@@ -277,3 +277,50 @@ def test_tq3_sink_and_window(dev, sub_n, num_q, sink, window):
     torch.cuda.synchronize()
     one, many = one.float().cpu().numpy(), many.float().cpu().numpy()
     assert np.isfinite(many).all() and rel_err(one, many) < TOL
+
+
+@pytest.mark.parametrize("fmt", ["tq3", "q8", "mixed"])
+def test_one_workspace_for_calls_of_every_kind(dev, fmt):
+    """One workspace in turn for one query, for a few and for many: each kind lays its
+    records out in its own way and leaves every tag clear for the next."""
+    import torch
+    make, call = _call(fmt)
+    num_q, num_kv, n_max = 16, 4, 6000
+    rng = np.random.default_rng(17)
+    kb, vb = _caches(rng, dev, fmt, n_max, num_kv)
+    ws = make(num_q, num_kv, 20, n_max, dev)
+    kw = dict(num_q=num_q, num_kv=num_kv, scale=1 / 16)
+    for n, sub_n in [(6000, 1), (5000, 16), (301, 1), (6000, 20), (4097, 3), (700, 12), (6000, 16), (6000, 1)]:
+        qd = _dev(q_f16(rng, sub_n, num_q, 256).view(np.uint16), dev).view(torch.float16)
+        got, want = torch.zeros_like(qd), torch.zeros_like(qd)
+        call(qd, kb, vb, got, ws, start_pos=n - sub_n, sub_n=sub_n, **kw)
+        call(qd, kb, vb, want, make(num_q, num_kv, 20, n_max, dev), start_pos=n - sub_n, sub_n=sub_n, **kw)
+        torch.cuda.synchronize()
+        assert torch.isfinite(got).all() and torch.equal(got, want), (n, sub_n)
+
+
+@pytest.mark.parametrize("fmt", ["tq3", "mixed"])
+@pytest.mark.parametrize("rows,scale", [(slice(100, 140), 40), (slice(1800, 1801), 2500), (slice(2990, 3000), 300)])
+def test_large_value_norms(dev, fmt, rows, scale):
+    """Block norms above 128 (here 500 to 50,000) end the slack of the reference maximum
+    from their tile on, so that weight x norm stays inside fp16; tiles before them were
+    taken with it."""
+    import torch
+    make, call = _call(fmt)
+    n, num_q, num_kv, sub_n = 3000, 16, 4, 12
+    rng = np.random.default_rng(scale)
+    k16, v16 = kv_f16(rng, n, num_kv, 256), kv_f16(rng, n, num_kv, 256).astype(np.float32)
+    v16[rows] = np.clip(v16[rows], -8, 8) * scale
+    kb = _dev((O.tq3_encode(k16) if fmt == "tq3" else O.q8_encode(k16)).view(np.uint8), dev)
+    vb = _dev(O.tq3_encode(v16.astype(np.float16)).view(np.uint8), dev)
+    q = (q_f16(rng, sub_n, num_q, 256).astype(np.float32) * np.linspace(0.5, 4, sub_n)[:, None, None]).astype(np.float16)
+    qd = _dev(q.view(np.uint16), dev).view(torch.float16)
+    ws = make(num_q, num_kv, sub_n, n, dev)
+    one, many = torch.zeros_like(qd), torch.zeros_like(qd)
+    kw = dict(num_q=num_q, num_kv=num_kv, scale=1 / 16)
+    call(qd, kb, vb, one, ws, start_pos=n - sub_n, sub_n=sub_n, **kw)
+    for t in range(sub_n):
+        call(qd[t:t + 1].contiguous(), kb, vb, many[t:t + 1], ws, start_pos=n - sub_n + t, sub_n=1, **kw)
+    torch.cuda.synchronize()
+    one, many = one.float().cpu().numpy(), many.float().cpu().numpy()
+    assert np.isfinite(many).all() and rel_err(one, many) < TOL

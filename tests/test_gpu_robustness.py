@@ -145,6 +145,46 @@ def test_q8_decode_merge_timeout(dev):
     _timeout_cycle(dev, call, ws, ref)
 
 
+@pytest.mark.parametrize("kind,n,sub_n", [
+    ("q8", 3000, 16), ("mixed", 3000, 16),   # the multi-query kernel, its records merged by a second launch
+    ("q8", 301, 12), ("mixed", 301, 12),     # one query per workgroup, as many units that a second launch merges
+    ("paged", 900, 6),                       # ragged slots, merged by a second launch
+])
+def test_second_launch_merge_timeout(dev, kind, n, sub_n):
+    """The merge that is a launch of its own takes a poll limit of 0 like the others."""
+    import torch
+    from qengine_amd import kvcache
+    rng = np.random.default_rng(75 + n + sub_n)
+    nq, nkv = 16, 4
+    q = q_f16(rng, sub_n, nq, 256)
+    k16, v16 = kv_f16(rng, n, nkv, 256), kv_f16(rng, n, nkv, 256)
+    kb = O.tq3_encode(k16) if kind == "paged" else O.q8_encode(k16)
+    vb = O.q8_encode(v16) if kind == "q8" else O.tq3_encode(v16)
+    qd, kd, vd = _dev(q.view(np.uint16), dev), _dev(kb.view(np.uint8), dev), _dev(vb.view(np.uint8), dev)
+    kw = dict(num_q=nq, num_kv=nkv, scale=1 / 16)
+    if kind == "paged":
+        ctx = np.array([n, 1, 500, 64, 65, 700][:sub_n], np.int32)
+        table = _dev(np.tile(np.arange((n + 63) // 64, dtype=np.int32), (sub_n, 1)), dev)
+        pool = [torch.zeros(((n + 63) // 64 * 64 * nkv * 2, 52), dtype=torch.uint8, device=dev) for _ in range(2)]
+        for x, y in zip(pool, (kd, vd)):
+            x.view(-1)[:y.numel()] = y.reshape(-1)
+        ws = kvcache.decode_attn_tq3_paged_workspace(nq, nkv, sub_n, n, dev)
+    else:
+        make = kvcache.decode_attn_q8_workspace if kind == "q8" else kvcache.decode_attn_q8k_tq3v_workspace
+        run = kvcache.decode_attn_q8 if kind == "q8" else kvcache.decode_attn_q8k_tq3v
+        ws = make(nq, nkv, sub_n, n, dev)
+
+    def call():
+        out = torch.zeros((sub_n, nq, 256), dtype=torch.float16, device=dev)
+        if kind == "paged":
+            kvcache.decode_attn_tq3_paged(qd.view(torch.float16), *pool, out, ws, table, _dev(ctx, dev), max_ctx=n,
+                                          block_tokens=64, **kw)
+        else:
+            run(qd, kd, vd, out, ws, start_pos=n - sub_n, sub_n=sub_n, **kw)
+        torch.cuda.synchronize()
+        return out.cpu().numpy().astype(np.float64)
+    _timeout_cycle(dev, call, ws, call())
+
 
 def test_noalloc_decode_merge_timeout(dev):
     """The allocation-free decode's scratch through its device-keyed status and

@@ -19,8 +19,12 @@ Q8_BLOCK_BYTES = 36
 
 
 def _stream(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    """The raw stream of `stream`, or of the current stream of the current device
+    (looked up as an integer: a torch.cuda.Stream object costs 2.7 us of a call's
+    host time, as much as a kernel launch)."""
+    if stream is not None:
+        return stream.cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 # fp16 arguments: torch.float16, or 16-bit integer tensors holding fp16 bit

@@ -341,14 +341,36 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   }
   __builtin_amdgcn_sched_barrier(0);
   // ---- key range of the workgroup
-  const int active_last = p.start_pos + t0 + nq;
+  const int active_last = __builtin_amdgcn_readfirstlane(p.start_pos + t0 + nq);
   int lo = chunk * p.chunk_keys;
   const int c_end = !SPLIT && chunk == p.n_chunks - 1 ? active_last : lo + p.chunk_keys;
   int hi = min(c_end, active_last), hi_first = min(c_end, p.start_pos + t0 + 1);
   lo = __builtin_amdgcn_readfirstlane(lo);
   hi = __builtin_amdgcn_readfirstlane(hi);
   hi_first = __builtin_amdgcn_readfirstlane(hi_first);
-  const int n_tiles = hi > lo ? (hi - lo + kTile - 1) / kTile : 0;
+  int n_tiles = hi > lo ? (hi - lo + kTile - 1) / kTile : 0;
+  // ---- the sink / window rule (KeyRule), by tile where all columns agree: the tiles
+  // that none sees (past the sink, before the first query's window) are one range, left
+  // out of the walk; of the others, those that every column sees need no rule.  (A
+  // branch in the loop instead of this cost calls without a sink or window 3 us of 84,
+  // 16 queries over 131,072 keys.)
+  const bool sw = KT && (p.sink_tok > 0 || p.window_tok > 0);
+  int skip_from = n_tiles, skip_keys = 0;
+  if (sw) {
+    const int seen_from = p.start_pos + t0 + 1 - p.window_tok;
+    const int first = p.sink_tok > lo ? (p.sink_tok - lo - 1) / kTile + 1 : 0;
+    const int past = seen_from > lo ? min(n_tiles, (seen_from - lo) / kTile) : 0;
+    if (past > first) {
+      skip_from = first;
+      skip_keys = (past - first) * kTile;
+      n_tiles -= past - first;
+    }
+  }
+  n_tiles = __builtin_amdgcn_readfirstlane(n_tiles);
+  skip_from = __builtin_amdgcn_readfirstlane(skip_from);
+  skip_keys = __builtin_amdgcn_readfirstlane(skip_keys);
+  auto tile_key = [&](int t) { return lo + t * kTile + (KT && t >= skip_from ? skip_keys : 0); };
+  auto sw_all = [&](int t32) { return t32 < p.sink_tok || t32 + 32 > active_last - p.window_tok; };
   // ---- fused append (qkv_decode_attn_tq3_append): the new keys start_pos ..
   // that this workgroup reads, [new_lo, new_lo + n_new), are encoded here
   // (tq3_encode_row16, the small append's arithmetic), 32 blocks per round, and
@@ -381,8 +403,8 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
 
   const uint32_t rows = mq_rows<KT, VT>(tid);
   MqRegs<KT, VT> ra, rb;
-  if (n_tiles > 0) mq_load<KT, VT>(p, lo, h, tid, wave, lane, rows, ra);
-  if (n_tiles > 1) mq_load<KT, VT>(p, lo + kTile, h, tid, wave, lane, rows, rb);
+  if (n_tiles > 0) mq_load<KT, VT>(p, tile_key(0), h, tid, wave, lane, rows, ra);
+  if (n_tiles > 1) mq_load<KT, VT>(p, tile_key(1), h, tid, wave, lane, rows, rb);
   const uint32_t lane4 = 4u * (uint32_t)lane;
   if constexpr (VT) {
     // table: wave w writes every lane's copy of entries 8 w .. 8 w + 7
@@ -461,11 +483,6 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   // tiles before this key are seen whole by every column, as far as the end of its keys
   // and the tree bits (keys past start_pos) go
   const int dense_end = KT && p.tree_mask != nullptr ? min(hi_first, p.start_pos) : hi_first;
-  // the sink / window rule on 32-key tiles (KeyRule), for all columns: seen by every one
-  // that has the whole tile among its keys, seen by none
-  const bool sw = KT && (p.sink_tok > 0 || p.window_tok > 0);
-  auto sw_all = [&](int t32) { return t32 < p.sink_tok || t32 + 32 > active_last - p.window_tok; };
-  auto sw_none = [&](int t32) { return t32 >= p.sink_tok && t32 + 32 <= p.start_pos + t0 + 1 - p.window_tok; };
   // (opaque thread indexes: the offsets of staging and loads are formed at each
   // use instead of being held in registers through the loop)
   auto stage = [&](int ts, int buf, MqRegs<KT, VT>& r) {
@@ -480,9 +497,9 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     mq_load<KT, VT>(p, ts, h, ti, wave, ti & 63, rows, r);
   };
   // tiles 0 and 1 staged, tile 2 on its way
-  if (n_tiles > 0) stage(lo, 0, ra);
-  if (n_tiles > 1) stage(lo + kTile, 1, rb);
-  if (n_tiles > 2) load(lo + 2 * kTile, ra);
+  if (n_tiles > 0) stage(tile_key(0), 0, ra);
+  if (n_tiles > 1) stage(tile_key(1), 1, rb);
+  if (n_tiles > 2) load(tile_key(2), ra);
   __syncthreads();
 
   // (a reference that no visible score has touched yet is kNoRef, not -inf: the
@@ -514,36 +531,14 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   // tile t's staging buffer and flag, those of t + 1 and of t + 2
   int b0 = 0, b1 = 1, b2 = 2;
   float slack = kSlack<VT>;
-  // behind a tile's barrier: tile t + 2 into the free buffer, t + 3 on its way
-  auto advance = [&](int ts, int t, int b2, MqRegs<KT, VT>& r) {
-    if constexpr (VT) slack = __builtin_amdgcn_readfirstlane(flag_s[3]) ? 0.0f : kSlack<VT>;
-    if (t + 2 < n_tiles) {
-      stage(ts + 2 * kTile, b2, r);
-      if (t + 3 < n_tiles) load(ts + 3 * kTile, r);
-    }
-    if (tid == 0) flag_s[b2] = 0;   // (set by tile t + 2, after the next barrier)
-  };
   for (int t = 0; t < n_tiles; t++) {
-    const int ts = lo + t * kTile;
+    const int ts = tile_key(t);
     const uint8_t* kbuf = lds + L::kK + b0 * L::kKBuf;
     const uint8_t* vbuf = lds + L::kV + b0 * L::kVBuf;
     const float* knorm = reinterpret_cast<const float*>(lds + L::kNorm) + b0 * 4 * kTile;
     uint8_t* pbuf = lds + L::kP + (t & 1) * L::kPBuf;
     bool dense = ts + kTile <= dense_end;
-    if constexpr (KT) {
-      if (sw) {
-        dense = dense && sw_all(ts) && sw_all(ts + 32);
-        if (sw_none(ts) && sw_none(ts + 32)) {   // nothing of it counts: only keep the pipeline going
-          __syncthreads();
-          advance(ts, t, b2, ra);
-          const int b = b0;
-          b0 = b1;
-          b1 = b2;
-          b2 = b;
-          continue;
-        }
-      }
-    }
+    if (KT && sw) dense = dense && sw_all(ts) && sw_all(ts + 32);
     bool v_nonfinite = false;
     if constexpr (!VT) {
       // the scales of this wave's value block, one key per lane, to the wave's own area
@@ -750,7 +745,12 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
           for (int r = 0; r < 4; r++) acc[g][e][r] *= cr[r];
       }
     }
-    advance(ts, t, b2, ra);
+    if constexpr (VT) slack = __builtin_amdgcn_readfirstlane(flag_s[3]) ? 0.0f : kSlack<VT>;
+    if (t + 2 < n_tiles) {
+      stage(tile_key(t + 2), b2, ra);
+      if (t + 3 < n_tiles) load(tile_key(t + 3), ra);
+    }
+    if (tid == 0) flag_s[b2] = 0;   // (set by tile t + 2, after the next barrier)
 #pragma unroll
     for (int cg = 0; cg < kCg; cg++) {
       lsum[cg] += ps[cg];

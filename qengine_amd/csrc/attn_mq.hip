@@ -280,10 +280,11 @@ __device__ __forceinline__ uint32_t pair_read(const uint8_t* lds, uint32_t w, ui
 // SPLIT: the split API.  The chunk is a reference split, whose partials (true maximum
 // in natural-log units, sum, unnormalised row in the caller's coordinates) go to
 // part_m / part_l / part_o.
-template <bool KT, bool VT, int NG, bool SPLIT>
+// SW: a sink or a window (TQ3 caches).
+template <bool KT, bool VT, int NG, bool SPLIT, bool SW = false>
 __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARAMS, AttnArgs pin) {
   QKV_ATTN_LEAD_APPLY(p, pin);
-  static_assert(!KT || VT, "TQ3 keys come with TQ3 values");
+  static_assert((!KT || VT) && (KT || !SW), "TQ3 keys come with TQ3 values, sinks and windows with TQ3 keys");
   using L = MqLds<KT, VT>;
   __shared__ __attribute__((aligned(16))) uint8_t lds[L::kEnd];
   const int tid = threadIdx.x;
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   }
   __builtin_amdgcn_sched_barrier(0);
   // ---- key range of the workgroup
-  const int active_last = __builtin_amdgcn_readfirstlane(p.start_pos + t0 + nq);
+  const int active_last = p.start_pos + t0 + nq;
   int lo = chunk * p.chunk_keys;
   const int c_end = !SPLIT && chunk == p.n_chunks - 1 ? active_last : lo + p.chunk_keys;
   int hi = min(c_end, active_last), hi_first = min(c_end, p.start_pos + t0 + 1);
@@ -351,25 +352,20 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
   int n_tiles = hi > lo ? (hi - lo + kTile - 1) / kTile : 0;
   // ---- the sink / window rule (KeyRule), by tile where all columns agree: the tiles
   // that none sees (past the sink, before the first query's window) are one range, left
-  // out of the walk; of the others, those that every column sees need no rule.  (A
-  // branch in the loop instead of this cost calls without a sink or window 3 us of 84,
-  // 16 queries over 131,072 keys.)
-  const bool sw = KT && (p.sink_tok > 0 || p.window_tok > 0);
-  int skip_from = n_tiles, skip_keys = 0;
-  if (sw) {
+  // out of the walk; of the others, those that every column sees need no rule.  (An
+  // instance of its own: even this much costs other calls 1%, a branch in the loop 3.5%:
+  // 16 queries over 131,072 keys 83.4, 84.1 and 87.0 us.)
+  int skip_from = 0, skip_keys = 0;
+  if constexpr (SW) {
     const int seen_from = p.start_pos + t0 + 1 - p.window_tok;
     const int first = p.sink_tok > lo ? (p.sink_tok - lo - 1) / kTile + 1 : 0;
     const int past = seen_from > lo ? min(n_tiles, (seen_from - lo) / kTile) : 0;
-    if (past > first) {
-      skip_from = first;
-      skip_keys = (past - first) * kTile;
-      n_tiles -= past - first;
-    }
+    const int out = __builtin_amdgcn_readfirstlane(max(past - first, 0));
+    skip_from = __builtin_amdgcn_readfirstlane(first);
+    skip_keys = out * kTile;
+    n_tiles -= out;
   }
-  n_tiles = __builtin_amdgcn_readfirstlane(n_tiles);
-  skip_from = __builtin_amdgcn_readfirstlane(skip_from);
-  skip_keys = __builtin_amdgcn_readfirstlane(skip_keys);
-  auto tile_key = [&](int t) { return lo + t * kTile + (KT && t >= skip_from ? skip_keys : 0); };
+  auto tile_key = [&](int t) { return lo + t * kTile + (SW && t >= skip_from ? skip_keys : 0); };
   auto sw_all = [&](int t32) { return t32 < p.sink_tok || t32 + 32 > active_last - p.window_tok; };
   // ---- fused append (qkv_decode_attn_tq3_append): the new keys start_pos ..
   // that this workgroup reads, [new_lo, new_lo + n_new), are encoded here
@@ -538,7 +534,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
     const float* knorm = reinterpret_cast<const float*>(lds + L::kNorm) + b0 * 4 * kTile;
     uint8_t* pbuf = lds + L::kP + (t & 1) * L::kPBuf;
     bool dense = ts + kTile <= dense_end;
-    if (KT && sw) dense = dense && sw_all(ts) && sw_all(ts + 32);
+    if constexpr (SW) dense = dense && sw_all(ts) && sw_all(ts + 32);
     bool v_nonfinite = false;
     if constexpr (!VT) {
       // the scales of this wave's value block, one key per lane, to the wave's own area
@@ -622,7 +618,7 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       int c = c0 + 16 * cg, k0 = ts;
       asm volatile("" : "+v"(c), "+s"(k0));
       const int tq = t0 + min(c / gqa, nq - 1), end = p.start_pos + tq + 1;
-      const KeyRule rule(p.start_pos, tq, KT ? p.sink_tok : 0, KT ? p.window_tok : 0, KT ? p.tree_mask : nullptr);
+      const KeyRule rule(p.start_pos, tq, SW ? p.sink_tok : 0, SW ? p.window_tok : 0, KT ? p.tree_mask : nullptr);
       uint32_t bits = 0u;
 #pragma unroll
       for (int r = 0; r < 4; r++) {
@@ -955,18 +951,21 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
 
 }  // namespace
 
-template <bool KT, bool VT>
+template <bool KT, bool VT, bool SW = false>
 static void launch_mq(const AttnArgs& a, int n_wg, hipStream_t stream) {
   if (a.qpw * (a.num_q / a.num_kv) > 32)
-    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 4, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
+    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 4, false, SW>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
   else
-    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 2, false>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
+    hipLaunchKernelGGL((mq_attn_kernel<KT, VT, 2, false, SW>), dim3(n_wg), dim3(kThreads), 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
 }
+static bool has_sink_or_window(const AttnArgs& a) { return a.sink_tok > 0 || a.window_tok > 0; }
 
 hipError_t launch_mq_attn(const AttnArgs& a, bool k_tq3, bool v_tq3, uint16_t* out, hipStream_t stream) {
   const int groups = (a.sub_n + a.qpw - 1) / a.qpw * a.n_chunks;
   const int n_wg = (groups + 7) / 8 * 8 * a.num_kv;
-  if (k_tq3)
+  if (k_tq3 && has_sink_or_window(a))
+    launch_mq<true, true, true>(a, n_wg, stream);
+  else if (k_tq3)
     launch_mq<true, true>(a, n_wg, stream);
   else if (v_tq3)
     launch_mq<false, true>(a, n_wg, stream);
@@ -982,7 +981,9 @@ hipError_t launch_mq_split(const AttnArgs& a, bool tq3, hipStream_t stream) {
   const dim3 grid((groups + 7) / 8 * 8 * a.num_kv), block(kThreads);
   const bool wide = a.qpw * (a.num_q / a.num_kv) > 32;
   if (tq3 && wide) return hipErrorInvalidValue;
-  if (tq3)
+  if (tq3 && has_sink_or_window(a))
+    hipLaunchKernelGGL((mq_attn_kernel<true, true, 2, true, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
+  else if (tq3)
     hipLaunchKernelGGL((mq_attn_kernel<true, true, 2, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a);
   else if (wide)
     hipLaunchKernelGGL((mq_attn_kernel<false, false, 4, true>), grid, block, 0, stream, QKV_ATTN_LEAD_ARGS(a), a);

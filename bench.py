@@ -334,9 +334,9 @@ def secondary(torch, kvcache, dev, stream):
         "prefill_path_us": round(ms_pf * 1e3, 3),
         "note": "append of the 16 verify tokens, then causal attention of the 16 queries over "
                 "the TQ3 cache (131088 keys, the block's own keys read back quantized), in one "
-                "call and one launch: qkv_decode_attn_tq3_append, whose decode kernel encodes "
-                "the block's rows itself, writes them to the caches and decodes every tile once "
-                "for all 64 query-head columns (caches and output bit-identical to the two "
+                "call: qkv_decode_attn_tq3_append, whose decode kernel encodes "
+                "the block's rows itself, writes them to the caches and reads every tile once "
+                "for all 64 query-head columns, and a second launch merges (caches and output bit-identical to the two "
                 "calls); two_call_us: qkv_tq3_append_kv, then qkv_decode_attn_tq3 with sub_n 16; "
                 "prefill_path_us: the same step through qkv_prefill_attn_tq3 in verify mode"}
 

@@ -282,13 +282,14 @@ int qkv_attn_split_merge(const float* part_m, const float* part_l, const float* 
 size_t qkv_decode_attn_tq3_workspace_bytes(int num_q, int num_kv, int sub_n, int n_keys);
 
 /* Fast path for the same computation as qkv_attn_split_tq3 + qkv_attn_split_merge
- * (model.cuh:2472-2491) in ONE launch: the key range is cut into chunks of
- * 512*k keys (the last one may also take a remainder of at most 64 keys),
- * partials stay in rotated coordinates and are merged inside the kernel (the
- * last workgroups of the grid do the merge), and each output row is rotated
- * back once.  The queries of a multi-token call (verify, sub_n > 1) share
+ * (model.cuh:2472-2491) in one call: the key range is cut into chunks (512*k
+ * keys, the last one maybe a remainder of at most 64 more; whole 64-key tiles
+ * with more than 16 (query, head) columns), partials stay in rotated
+ * coordinates and are merged inside the kernel (the last workgroups of the
+ * grid do the merge) or, with many rows, by a second launch, and each output
+ * row is rotated back once.  The queries of a multi-token call (verify, sub_n > 1) share
  * passes over the cache: up to 16 (query, head) columns per pass, and calls
- * with more columns decode each tile once for up to 64 of them.
+ * with more columns read each tile once for up to 64 of them.
  * out [sub_n][num_q][256] fp16 (16-byte aligned).
  * workspace: caller-owned device memory of at least
  * qkv_decode_attn_tq3_workspace_bytes() bytes, 256-byte aligned, ZERO-FILLED
@@ -306,7 +307,8 @@ int qkv_decode_attn_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_blo
  * a bounded poll; if the bound runs out (a launch starved of GPU time for
  * seconds), the affected output rows are written as NaN and the workspace
  * header keeps an error word, after which every later call on that workspace
- * writes NaN rows until it is reset.  No counterpart in the reference (its
+ * writes NaN rows until it is reset.  (A call whose merge is a second launch
+ * does not wait, and reports a record that is missing there in the same way.)  No counterpart in the reference (its
  * merge is a separate launch, attention.cuh:1837-1891).
  * qkv_decode_workspace_status synchronises `stream`, then returns QKV_OK or
  * QKV_ERR_TIMEOUT.  qkv_decode_workspace_reset zero-fills `bytes` bytes of
@@ -337,11 +339,11 @@ int qkv_debug_set_merge_spin_limit(int limit);
  * fp16 K and V rows [sub_n][num_kv][256] (16-byte aligned); they are encoded
  * exactly as qkv_tq3_append_kv encodes them and written to rows start_pos ..
  * start_pos + sub_n - 1 of k and v, and the attention is that of
- * qkv_decode_attn_tq3 with the same arguments.  It is ONE launch for a
- * decode step (sub_n = 1: the wave whose tile holds the new key encodes it)
- * and for calls with more than 16 (query, head) columns and sub_n <= 64 (the
- * shared-decode kernel encodes the new rows it reads); both write the rows to
- * the caches.  Other shapes take the append's launch, then the decode's.  Caches and output equal those of
+ * qkv_decode_attn_tq3 with the same arguments.  The append needs no launch of
+ * its own for a decode step (sub_n = 1: the wave whose tile holds the new key
+ * encodes it) and for calls with more than 16 (query, head) columns and sub_n
+ * <= 64 (the multi-query kernel encodes the new rows it reads); both write the
+ * rows to the caches.  Other shapes take the append's launch first.  Caches and output equal those of
  * qkv_tq3_append_kv followed by qkv_decode_attn_tq3; same workspace
  * (qkv_decode_attn_tq3_workspace_bytes(num_q, num_kv, sub_n,
  * start_pos + sub_n)) and errors. */
@@ -359,9 +361,9 @@ int qkv_decode_attn_tq3_append(const uint16_t* q, const uint16_t* k_new, const u
  * each GPU it runs on until the process ends; the call itself allocates
  * nothing.  qkv_tq3_init(device) looks the array up and zero-fills it (so
  * does the first call on a device if init was not called; it also re-clears
- * it, the reset after a merge timeout).  Shapes whose workspace
- * (qkv_decode_attn_tq3_workspace_bytes) exceeds 8 MiB return
- * QKV_ERR_WORKSPACE.  Every call on one GPU shares that GPU's scratch, which
+ * it, the reset after a merge timeout).  Shapes whose records do not fit
+ * 8 MiB (with more than 16 (query, head) columns: with chunks of 512 keys or
+ * longer) return QKV_ERR_WORKSPACE.  Every call on one GPU shares that GPU's scratch, which
  * each completed call leaves ready for the next: calls that overlap on one
  * GPU (different streams, or a concurrent qkv_tq3_init) race and must not be
  * issued. */
@@ -384,9 +386,10 @@ int qkv_decode_noalloc_status_async(int device, int* status, hipStream_t stream)
 int qkv_decode_noalloc_reset(int device, hipStream_t stream);
 
 /* Fast path for qkv_attn_split_q8 + qkv_attn_split_merge over the Q8_0 cache
- * (decode launch model.cuh:2430-2463; attention.cuh:2633-2801 and 1837-1891) in ONE launch:
- * chunks of 128*k keys, records merged inside the kernel as for
- * qkv_decode_attn_tq3 (values are not rotated).  Same argument meaning as
+ * (decode launch model.cuh:2430-2463; attention.cuh:2633-2801 and 1837-1891) in one call:
+ * chunks of 128*k keys, records merged inside the kernel (calls of many
+ * queries: by a second launch) as for qkv_decode_attn_tq3 (values are not
+ * rotated).  Same argument meaning as
  * qkv_attn_split_q8 (no sink/window/tree rules, as in the reference) with the
  * merged fp16 output and a workspace of qkv_decode_attn_q8_workspace_bytes()
  * bytes (256-byte aligned, zero-filled before first use, reused in order). */

@@ -37,11 +37,11 @@ struct AttnArgs {
   uint64_t v_bytes;         // value cache extent when its format differs from the keys' (else unused)
   int num_q, num_kv;
   int start_pos, sub_n, sub_n_max;
-  int qpw;                  // queries per workgroup (MFMA columns = qpw * gqa <= 16)
+  int qpw;                  // queries per workgroup (MFMA columns = qpw * gqa <= 16, in attn_mq.hip <= 64)
   int active_end_max;       // reference split sizing (split API)
   int k_splits;             // reference split count (split API)
   int n_chunks;             // workgroups per (kv head, query group): k_splits or key chunks
-  int chunk_keys;           // keys per fast-path chunk (multiple of 256)
+  int chunk_keys;           // keys per fast-path chunk (whole 64-key tiles; Q8_0, one query per workgroup: 128)
   int n_slots;              // fast-path records per (q head, query): n_chunks
   float scale_log2;         // softmax scale * log2(e)
   int sink_tok, window_tok;

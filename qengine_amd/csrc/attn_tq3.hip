@@ -20,15 +20,16 @@
 //           share the 16 columns, or, for calls with more than 8 / GQA
 //           queries, fill them with 16 / GQA queries each, the remainders
 //           read from LDS into a second product chained onto the first):
-//           lane (key, octet o) reads the 12 aligned bytes holding
-//           code groups 4o..4o+3 of each 128-block and decodes centroid pairs
-//           through a per-lane LDS table.  One accumulator per 128-block, each
+//           lane (key, octet o) takes the 12 bytes holding code groups
+//           4o..4o+3 of each 128-block and decodes centroid pairs through a
+//           per-lane LDS table.  The fast path loads a tile in 16-byte units,
+//           four lanes to a block, and passes the keys through LDS (TileRegs);
+//           the split forms load each lane's own 12 bytes (TileRows).  One accumulator per 128-block, each
 //           scaled by its block norm (which carries the softmax scale).
 //   softmax online, per head, base 2.
 //   values  v_mfma_f32_16x16x32_f16, A = p*norm (fp16, the lane's own
-//           probabilities), B = codes of 32 keys x 16 dims.  The wave's value
-//           rows are loaded with aligned 16-byte loads (lane = key) and staged
-//           in LDS; lane (n, o) gathers dim group n of both blocks for 8 keys
+//           probabilities), B = codes of 32 keys x 16 dims.  The value codes
+//           are staged in LDS, a dword per dim group and key; lane (n, o) gathers dim group n of both blocks for 8 keys
 //           and interleaves the codes of key pairs (bit select), so that each
 //           table entry read is a B dword (two keys, one dim); the table
 //           reads run two steps ahead.
@@ -37,9 +38,8 @@
 // workgroup's data stores are complete.  The last workgroups of the grid are
 // designated mergers, one per (q head, query, 128-block) unit: each polls its
 // unit's tags (bounded), clears them, reads the rows in one round of 16-byte
-// loads, merges, rotates back and stores fp16 (attn_fastmerge.h).  Only
-// mergers wait, so progress does not depend on workgroup co-residency.  Paged
-// (ragged) launches split each kv head's record shares over the slots in
+// loads, merges, rotates back and stores fp16 (attn_fastmerge.h); calls with
+// many units leave that to a second launch (merges_apart).  Paged (ragged) launches split each kv head's record shares over the slots in
 // proportion to their key counts.  Split API: one workgroup per reference
 // split, written in the reference partial layout.
 #include <algorithm>
@@ -1018,7 +1018,7 @@ __global__ __launch_bounds__(kThreads, 1) void tq3_attn_kernel(QKV_ATTN_LEAD_PAR
   lsum = xrow_sum(lsum);
   QKV_STAMP(kPhTiles);
 
-  // ---------------- merge the 4 waves in LDS ----------------
+  // ---------------- merge the waves in LDS ----------------
   __syncthreads();
   QKV_STAMP(kPhTileBar);
   float* mo = reinterpret_cast<float*>(lds + kLdsMergeO);    // [wave][8][256]

@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256) void prefill_stage_small_kernel(PrefillArgs p,
 constexpr long kStSmallWgs = 512;   // 64-row tiles x kv heads up to which the small form is launched
 
 // ---------------------------------------------------------------------------
-// attention: 1-D grid (placement above); WAVES query heads of one kv head and
+// attention: 1-D grid (Sched, above); WAVES query heads of one kv head and
 // TG groups of 32 query tokens per workgroup, one wave per (head, group)
 // ---------------------------------------------------------------------------
 template <int WAVES, int TG, bool FROM_CACHE>

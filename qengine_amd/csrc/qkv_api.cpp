@@ -794,7 +794,7 @@ static int decode_tq3(const uint16_t* q, const qkv_block_tq3* k, const qkv_block
   a.ws_o_bytes = (uint32_t)(g.total - g.o_off);
   if (k_new) {
     // the block's rows start_pos .. start_pos + sub_n - 1: encoded inside the
-    // decode launch when it takes the shared-decode kernel (more than 16
+    // decode launch when it takes the multi-query kernel (more than 16
     // query-head columns) and the block has at most 64 rows (the kernel's
     // encode area: a workgroup encodes the new rows it reads, at most
     // min(sub_n, 64)), or when it is one query (a decode step: the wave whose

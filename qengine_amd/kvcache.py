@@ -330,7 +330,7 @@ def decode_attn_tq3_workspace(num_q, num_kv, sub_n, n_keys, device) -> torch.Ten
 
 def decode_attn_tq3(q, k, v, out, workspace, *, num_q, num_kv, start_pos, sub_n, scale,
                     sink_tok=0, window_tok=0, tree_mask=None, head_dim=256, stream=None) -> None:
-    """Fast path: split-K decode with the merge inside the same launch."""
+    """Fast path: split-K decode and its merge in one call."""
     _attn_sizes(q, k, v, out, num_q, num_kv, start_pos + sub_n, sub_n, head_dim, TQ3_ROW, TQ3_ROW)
     check(lib().qkv_decode_attn_tq3(
         _dev_ptr(q, "q"), _dev_ptr(k, "k"), _dev_ptr(v, "v"), _dev_ptr(out, "out"), num_q,
@@ -344,8 +344,8 @@ def decode_attn_tq3_append(q, k_new, v_new, k, v, out, workspace, *, num_q, num_
                            stream=None) -> None:
     """decode_attn_tq3 of a block of sub_n new tokens whose K / V rows (fp16
     [sub_n][num_kv][256]) are appended in the same call: encoded into rows
-    start_pos .. start_pos + sub_n - 1 of k / v (one launch when the call has
-    more than 16 query-head columns).  k and v must hold those rows."""
+    start_pos .. start_pos + sub_n - 1 of k / v (inside the decode launch for one
+    query, and with more than 16 query-head columns).  k and v must hold those rows."""
     _attn_sizes(q, k, v, out, num_q, num_kv, start_pos + sub_n, sub_n, head_dim, TQ3_ROW, TQ3_ROW)
     _need(k_new, sub_n * num_kv * head_dim * 2, "k_new", FP16)
     _need(v_new, sub_n * num_kv * head_dim * 2, "v_new", FP16)

@@ -22,7 +22,7 @@ def _dev(a, dev):
 
 # (start_pos, num_q, sub_n, tree); num_kv 4, so sub_n * num_q / 4 (query, head) columns
 SHAPES = [
-    (32768, 16, 16, False),   # config 5(ii)'s block over 32K keys: 64 columns, one launch
+    (32768, 16, 16, False),   # config 5(ii)'s block over 32K keys: 64 columns, encoded in the decode launch
     (3000, 16, 16, True),     # tree mask
     (2500, 24, 16, False),    # 96 columns: two query groups; the last group stores the rows
     (2500, 32, 16, True),     # GQA 8, 128 columns: two query groups of 8 queries, tree mask

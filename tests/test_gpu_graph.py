@@ -133,7 +133,7 @@ def test_q8_append_and_decode_graph_replays(dev):
 
 def test_tq3_verify_append_in_decode_graph_replays(dev):
     """A 16-token verify block appended inside the decode launch
-    (qkv_decode_attn_tq3_append, one launch at 64 query-head columns) in a
+    (qkv_decode_attn_tq3_append, at 64 query-head columns) in a
     graph: every replay rewrites the block's cache rows with the same bytes
     and yields the eager output, with an eager decode of another shape on the
     same workspace between the replays."""

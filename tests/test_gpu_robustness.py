@@ -93,10 +93,8 @@ def test_tq3_decode_merge_timeout(dev):
 
 @pytest.mark.parametrize("sub_n", [16, 5])
 def test_tq3_multi_query_merge_timeout(dev, sub_n):
-    """The shared-decode multi-query path (more than 16 query-head columns):
-    its mergers take their units two at a time (16 queries: 16 units per
-    merger, all in pairs; 5 queries: 5 per merger, two pairs and a single),
-    and a timed-out pair writes NaN rows like a single unit."""
+    """The multi-query path (more than 16 query-head columns): its records are
+    merged by a second launch, which writes NaN rows like a timed-out merger."""
     import torch
     from qengine_amd import kvcache
     rng = np.random.default_rng(73 + sub_n)

@@ -662,8 +662,9 @@ size_t fast_ws_upto(int num_q, int num_kv, int sub_n, int n_keys, int base, int 
 // mq_attn_kernel (attn_mq.hip): queries per workgroup (returned) and chunks.
 // Chunks are whole 64-key tiles, at least two (a chunk pays for its records),
 // at most max_chunks of them; the launch is one round of the GPU, or one chunk
-// per (query group, kv head) where these alone are more.  A call that leaves CUs idle is split over query groups: fewer columns make a tile cheaper
-// and leave each workgroup fewer record rows to write.
+// per (query group, kv head) where these alone are more.  A call that leaves CUs
+// idle is split over query groups: fewer columns make a tile cheaper and leave
+// each workgroup fewer record rows to write.
 // Costs as measured (131,072 against 65,000 keys): 1.7 us per tile up to 32
 // columns, 2.05 with 64; 64 KB of records per workgroup ~3.2 us.
 int mq_geom(FastGeom& g, int num_q, int num_kv, int sub_n, int n_keys, int max_chunks) {

@@ -787,10 +787,11 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
         }
       }
     };
-    if (!VT && v_nonfinite && !dense) {
-      // a key that some query of the block does not see may have an inf or NaN
-      // scale: 0 * inf must not reach that query's rows, so every query takes
-      // products of its own, with the keys that it does not see zeroed
+    if (!VT && v_nonfinite) {
+      // a key with an inf or NaN scale: 0 * inf must not reach the rows of a query
+      // that does not see it, nor 0 be the rest of a weight there, so every query
+      // takes products of its own, of the weights alone, with the keys that it does
+      // not see zeroed
 #pragma unroll 1
       for (int it = 0; it < 2 * nq; it++) {
         const int c2 = it & 1, qi = it >> 1;
@@ -822,20 +823,17 @@ __global__ __launch_bounds__(kThreads, 1) void mq_attn_kernel(QKV_ATTN_LEAD_PARA
       for (int c2 = 0; c2 < 2; c2++) {
         u4_t bv[2];
         v_operands(c2, bv);
-        auto product = [&](int rest) {
+#pragma unroll
+        for (int part = 0; part < (VT ? 1 : 2); part++) {   // Q8_0 values: the weights, then their rests
           h8_t pa[NG];
 #pragma unroll
-          for (int g = 0; g < NG; g++) pa[g] = p_operand(g, c2, rest);
+          for (int g = 0; g < NG; g++) pa[g] = p_operand(g, c2, part);
 #pragma unroll
           for (int g = 0; g < NG; g++)
 #pragma unroll
             for (int e = 0; e < 2; e++)
               acc[g][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pa[g], __builtin_bit_cast(h8_t, bv[e]), acc[g][e], 0, 0, 0);
-        };
-        product(0);
-        // (with an inf scale the weights' rests, 0 among them, would make NaN of inf)
-        if constexpr (!VT)
-          if (!v_nonfinite) product(1);
+        }
       }
     }
     const int b = b0;

@@ -324,3 +324,17 @@ def test_large_value_norms(dev, fmt, rows, scale):
     torch.cuda.synchronize()
     one, many = one.float().cpu().numpy(), many.float().cpu().numpy()
     assert np.isfinite(many).all() and rel_err(one, many) < TOL
+
+
+def test_non_finite_value_scale_in_a_whole_tile(dev):
+    """An inf in a value row of the history, which every query sees: the same elements
+    are non-finite as in single-query calls, the others as near to them as ever."""
+    n, num_q, num_kv, sub_n = 4300, 16, 4, 16
+    rng = np.random.default_rng(6)
+    k16, v16 = kv_f16(rng, n, num_kv, 256), kv_f16(rng, n, num_kv, 256)
+    v16[1500, 2, 77] = np.inf
+    kb, vb = (_dev(O.q8_encode(x).view(np.uint8), dev) for x in (k16, v16))
+    one, many = _both(dev, "q8", q_f16(rng, sub_n, num_q, 256), kb, vb, n, num_q, num_kv)
+    bad = ~np.isfinite(many)
+    assert bad.any() and np.array_equal(bad, ~np.isfinite(one))
+    assert rel_err(np.where(bad, 0.0, one), np.where(bad, 0.0, many)) < TOL
